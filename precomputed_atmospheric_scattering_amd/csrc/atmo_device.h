@@ -138,6 +138,7 @@ struct Job {
   // which start at S64, SM64 and E_it, into S, SM and E.
   int acc64;
   int niter;
+  int it;  // Precompute iteration of the job, in [0, niter)
   // Optical depths of the transmittance texels (4 doubles per texel: the
   // Rayleigh, Mie and absorption density integrals), shared by the jobs of
   // one model: they depend on the geometry and density profiles only, not

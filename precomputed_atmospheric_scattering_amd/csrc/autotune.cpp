@@ -185,8 +185,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
   TUNE_HIP(hipEventCreate(&d.start));
   TUNE_HIP(hipEventCreate(&d.stop));
   const int w = z.nnu * z.nmus;
-  auto time_pass = [&](Pass pass, int order, int tile, int row_order,
-                       float* best) -> atmo_status {
+  auto time_pass = [&](Pass pass, int tile, int row_order, float* best) -> atmo_status {
     std::vector<atmo::Job> js(k);
     std::vector<int> fb(k + 1);
     int total = 0;
@@ -213,9 +212,11 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     pl.max_lds_w = w <= atmo::kMsMaxRow ? w : 0;
     pl.kinds = atmo::kJobsF32;
     pl.dj_kinds = atmo::kDjF32;
+    pl.arc_kinds = 0;
+    pl.arc_lds = 0;
     pl.tile = tile;
     auto launch = [&]() {
-      return pass == kSD ? atmo::launch_scattering_density(pl, order, s)
+      return pass == kSD ? atmo::launch_scattering_density(pl, s)
                          : atmo::launch_multiple_scattering(pl, s);
     };
     ATMO_TRY(check_launch(launch(), "tuning launch"));  // warm-up
@@ -238,14 +239,11 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     return t[dflt] >= kMinGain * t[best] ? best : dflt;
   };
   if (do_sd) {
-    // One order-2 launch and (for the default 4 orders) two higher-order
-    // launches per Init: the order-2 kernel also reads the single-Mie LUT.
     std::vector<double> t(atmo::kSdTiles);
     for (int tile = 0; tile < atmo::kSdTiles; ++tile) {
-      float t2 = 0.0f, t3 = 0.0f;
-      ATMO_TRY(time_pass(kSD, 2, tile, 0, &t2));
-      ATMO_TRY(time_pass(kSD, 3, tile, 0, &t3));
-      t[tile] = t2 + 2.0 * t3;
+      float ts = 0.0f;
+      ATMO_TRY(time_pass(kSD, tile, 0, &ts));
+      t[tile] = ts;
     }
     *sd_out = pick(t, atmo::sd_default_tile(z.nmu, z.nnu));
   }
@@ -261,7 +259,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
       if (w > atmo::kMsMaxRow && tile != dflt.tile) continue;
       for (int o = 0; o < kO; ++o) {
         float tm = 0.0f;
-        ATMO_TRY(time_pass(kMS, 0, tile, o, &tm));
+        ATMO_TRY(time_pass(kMS, tile, o, &tm));
         t[kO * tile + o] = tm;
       }
     }

@@ -24,6 +24,8 @@ struct PassLaunch {
   int tile;     // tile shape of the jobs (scattering density, multiple
                 // scattering): every job of a launch has the same one
   int dj_kinds;  // kDjF32 | kDjRgb21: the delta J formats of the jobs
+  int arc_kinds;   // arc_kind of the jobs, or-ed
+  size_t arc_lds;  // largest arc_lds of the jobs
 };
 
 constexpr int kDjF32 = 1;    // delta J as RGB float (FP32-storage jobs)
@@ -39,8 +41,8 @@ constexpr int kBlock = 256;
 // with the same operations in the same order, so the LUTs do not depend on
 // the choice.
 //
-// Scattering density: nu outputs per thread (they share the phase function
-// of the outgoing direction) and threads per block. A (r, mu_s) plane of
+// Scattering density of order 2: nu outputs per thread (they share the phase
+// function of the outgoing direction) and threads per block. A (r, mu_s) plane of
 // MU x ceil(NU / chunk) threads is split into ceil(plane / block) blocks,
 // each of which builds the plane's nu tables in LDS.
 struct SdTile {
@@ -52,11 +54,37 @@ constexpr SdTile kSdTile[kSdTiles] = {{4, 256}, {2, 256}, {1, 256},
 // Default shape: 4 nu per thread, in blocks of 128 threads when a plane has
 // at most 256 threads (MU x ceil(NU / 4)), else 256. Measured on MI355X
 // with the other shapes: at MU x NU = 128 x 8 (a 256-thread plane) the
-// 128-thread blocks are 4% faster at every order; at 256 x 16 (1024) the
+// 128-thread blocks are 4% faster; at 256 x 16 (1024) the
 // 256-thread blocks are, the blocks then rebuilding a plane's tables from
 // a LUT beyond the caches 4 times instead of 8.
 ATMO_HD int sd_default_tile(int nmu, int nnu) {
   return nmu * ((nnu + 3) / 4) <= 256 ? 3 : 0;
+}
+
+// Scattering density of orders >= 3 (density_arcs.h): a block of 8 waves
+// takes arc_cols mu_s columns and arc_mus mu rows of a layer, for the
+// wavelengths of up to kArcIters Precompute iterations. Each wave has
+// arc_tiles tiles of 64 (mu, nu) texels of a column: 512 rows of 2 columns,
+// 256 of 4, or 128 or 64 of 8, so that the source texels of an angle (cols x
+// kArcIters x NU) are at most one per thread. At most kArcMus mu rows' prefix
+// sums fit a block's LDS: 13/16 of the rows or more have texels from NU = 7 on
+// (all at 8, 16 and 32), 1/2 to 1 below.
+constexpr int kArcMaxCols = 8;
+constexpr int kArcMus = 16;
+constexpr int kArcIters = 5;
+ATMO_HD int arc_cols(int nnu) { return nnu >= 26 ? 2 : (nnu >= 13 ? 4 : 8); }
+ATMO_HD int arc_tiles(int nnu) { return nnu * kArcMus > 64 ? 2 : 1; }
+ATMO_HD int arc_mus(int nnu) {
+  const int mus = 8 / arc_cols(nnu) * arc_tiles(nnu) * 64 / nnu;
+  return mus < kArcMus ? mus : kArcMus;
+}
+// The instance that serves a job: its tiles per wave and the groups of 4
+// wavelengths of its iterations (those of the kArcIters from j.it on).
+ATMO_HD int arc_kind_bit(int tiles, int groups) { return 1 << (4 * (tiles - 1) + groups - 1); }
+ATMO_HD int arc_kind(const Job& j) {
+  const int left = j.niter - j.it;
+  const int nit = left < kArcIters ? left : kArcIters;
+  return arc_kind_bit(arc_tiles(j.nnu), (3 * nit + 3) / 4);
 }
 
 // Multiple scattering: packed rows of at most kMsMaxRow texels are processed
@@ -116,6 +144,8 @@ int blocks_transmittance(const Job& j);
 int blocks_direct_irradiance(const Job& j);
 int blocks_single_scattering(const Job& j);
 int blocks_scattering_density(const Job& j);
+int blocks_density_arcs(const Job& j);
+size_t arc_lds(const Job& j);  // LDS bytes of a block of launch_density_arcs
 int blocks_indirect_irradiance(const Job& j);
 int blocks_multiple_scattering(const Job& j);
 int blocks_half_conversion(const Job& j);
@@ -128,9 +158,11 @@ hipError_t launch_optical_depth(const PassLaunch& p, hipStream_t s);
 hipError_t launch_transmittance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_direct_irradiance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s);
-// 'order' is the scattering order being computed (>= 2).
-hipError_t launch_scattering_density(const PassLaunch& p, int order,
-                                     hipStream_t s);
+// The scattering density of order 2, and that of an order >= 3. In the
+// latter the jobs of a model's Precompute iterations follow each other in
+// p.jobs, and the blocks of the first of every kArcIters serve all of them.
+hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s);
+hipError_t launch_density_arcs(const PassLaunch& p, hipStream_t s);
 // 'order' is the order of the scattering read by the pass (>= 1).
 hipError_t launch_indirect_irradiance(const PassLaunch& p, int order,
                                       hipStream_t s);

@@ -10,87 +10,12 @@
 #include <type_traits>
 
 #include "atmo_device.h"
+#include "density_arcs.h"
 #include "kernels.h"
+#include "pass_common.h"
 
 namespace atmo {
 namespace {
-
-// Workgroups are dispatched to the 8 XCDs (each with its own L2) round-robin
-// by workgroup id. This permutation of a job's nb blocks gives the blocks of
-// one XCD (same id mod 8) a contiguous range of the job's work, so that the
-// blocks resident on an XCD at a time work on neighbouring rows and share
-// their L2 lines.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_contiguous(int lb, int nb) {
-  const int q = nb / kXcds, rem = nb % kXcds;
-  const int g = lb % kXcds;
-  return g * q + (g < rem ? g : rem) + lb / kXcds;
-}
-
-// Block b's job: the i with first_block[i] <= b < first_block[i + 1]. The
-// search is uniform across the block.
-__device__ __forceinline__ int find_job(const int* __restrict__ first_block,
-                                        int njobs, int b) {
-  int lo = 0, hi = njobs;
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (first_block[mid] <= b) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
-
-__device__ __forceinline__ float rcp_f(float x) {
-  return __builtin_amdgcn_rcpf(x);
-}
-__device__ __forceinline__ float rsq_f(float x) {
-  return __builtin_amdgcn_rsqf(x);
-}
-__device__ __forceinline__ float sqrt_f(float x) {
-  return __builtin_amdgcn_sqrtf(x);
-}
-__device__ __forceinline__ float clampf(float x, float lo, float hi) {
-  return fminf(fmaxf(x, lo), hi);
-}
-
-// cos and sin of (m + 1/2) * pi / 16 for m = 0..15, evaluated at compile time
-// (Taylor series in FP64, converged to the last bit for |x| <= pi).
-constexpr double cx_sin(double x) {
-  double term = x, sum = x;
-  for (int n = 1; n < 24; ++n) {
-    term *= -x * x / ((2.0 * n) * (2.0 * n + 1.0));
-    sum += term;
-  }
-  return sum;
-}
-constexpr double cx_cos(double x) {
-  double term = 1.0, sum = 1.0;
-  for (int n = 1; n < 24; ++n) {
-    term *= -x * x / ((2.0 * n - 1.0) * (2.0 * n));
-    sum += term;
-  }
-  return sum;
-}
-#define ATMO_PHI(m) ((m + 0.5) * 3.14159265358979323846 / 16.0)
-__device__ constexpr float kCosPhi[16] = {
-    float(cx_cos(ATMO_PHI(0))),  float(cx_cos(ATMO_PHI(1))),
-    float(cx_cos(ATMO_PHI(2))),  float(cx_cos(ATMO_PHI(3))),
-    float(cx_cos(ATMO_PHI(4))),  float(cx_cos(ATMO_PHI(5))),
-    float(cx_cos(ATMO_PHI(6))),  float(cx_cos(ATMO_PHI(7))),
-    float(cx_cos(ATMO_PHI(8))),  float(cx_cos(ATMO_PHI(9))),
-    float(cx_cos(ATMO_PHI(10))), float(cx_cos(ATMO_PHI(11))),
-    float(cx_cos(ATMO_PHI(12))), float(cx_cos(ATMO_PHI(13))),
-    float(cx_cos(ATMO_PHI(14))), float(cx_cos(ATMO_PHI(15)))};
-__device__ constexpr float kSinPhi[16] = {
-    float(cx_sin(ATMO_PHI(0))),  float(cx_sin(ATMO_PHI(1))),
-    float(cx_sin(ATMO_PHI(2))),  float(cx_sin(ATMO_PHI(3))),
-    float(cx_sin(ATMO_PHI(4))),  float(cx_sin(ATMO_PHI(5))),
-    float(cx_sin(ATMO_PHI(6))),  float(cx_sin(ATMO_PHI(7))),
-    float(cx_sin(ATMO_PHI(8))),  float(cx_sin(ATMO_PHI(9))),
-    float(cx_sin(ATMO_PHI(10))), float(cx_sin(ATMO_PHI(11))),
-    float(cx_sin(ATMO_PHI(12))), float(cx_sin(ATMO_PHI(13))),
-    float(cx_sin(ATMO_PHI(14))), float(cx_sin(ATMO_PHI(15)))};
-#undef ATMO_PHI
 
 // ---------------------------------------------------------------------------
 // Transmittance (functions.glsl:275-320, :454-463). FP64 throughout: the
@@ -472,8 +397,6 @@ __global__ __launch_bounds__(kBlock) void k_single_scattering(
 // direction. Ground-hitting theta_l add the ground-reflected term read from a
 // table of delta-irradiance row 0 (r = rb).
 // ---------------------------------------------------------------------------
-constexpr int kTheta = 16;
-
 // A table of n values v[0..n-1] has n + 1 entries of two float4:
 // (v.x, v.y, v.z, dv.x), (dv.y, dv.z, -, -). Entry 0 is a guard holding v[0]
 // with dv = 0; entry k >= 1 holds v[k - 1] with dv = v[k] - v[k - 1], and
@@ -511,7 +434,7 @@ struct SdTheta {
 // mu_s; consecutive nu) of a thread. The phase function of the scattering
 // towards the view direction depends on (mu, theta_l, phi) only, so it is
 // computed once per azimuth pair for all kChunk outputs.
-template <int kChunk, bool kOrder2, bool kGround>
+template <int kChunk, bool kGround>
 __device__ __forceinline__ void sd_theta(
     const float4* __restrict__ tab_a, const float4* __restrict__ tab_b,
     const float4* __restrict__ etab, float nu_max, float e_max, float A, float P,
@@ -557,37 +480,32 @@ __device__ __forceinline__ void sd_theta(
       for (int sgn = 0; sgn < 2; ++sgn) {
         const float t = sgn == 0 ? fmaf(tC[j], s, tb) : fmaf(-tC[j], s, tb);
         float3 v = table_lerp(tab_a, t);
-        float x1 = 1.0f;  // order 2: the Rayleigh phase factor 1 + nu1^2
-        if (kOrder2) {
-          // Order-1 incident radiance: Rayleigh and Mie single scattering
-          // times their phase functions of nu1 (constants folded in tables).
-          const float nu1 = fmaf(t, inv_hn, nu1_0);
-          const float3 vm = table_lerp(tab_b, t);
-          const float r1 = rsq_f(fmaf(mg2, nu1, g1));
-          const float q = r1 * r1 * r1;
-          x1 = fmaf(nu1, nu1, 1.0f);
-          v.x = fmaf(vm.x, q, v.x);
-          v.y = fmaf(vm.y, q, v.y);
-          v.z = fmaf(vm.z, q, v.z);
-        }
+        // Order-1 incident radiance: Rayleigh and Mie single scattering
+        // times their phase functions of nu1 (constants folded in tables);
+        // x1 is the factor 1 + nu1^2 of both.
+        const float nu1 = fmaf(t, inv_hn, nu1_0);
+        const float3 vm = table_lerp(tab_b, t);
+        const float r1 = rsq_f(fmaf(mg2, nu1, g1));
+        const float q = r1 * r1 * r1;
+        const float x1 = fmaf(nu1, nu1, 1.0f);
+        v.x = fmaf(vm.x, q, v.x);
+        v.y = fmaf(vm.y, q, v.y);
+        v.z = fmaf(vm.z, q, v.z);
         if (kGround) {
-          if (kOrder2) {
-            v.x = x1 * v.x;
-            v.y = x1 * v.y;
-            v.z = x1 * v.z;
-            x1 = 1.0f;
-          }
+          v.x = x1 * v.x;
+          v.y = x1 * v.y;
+          v.z = x1 * v.z;
           const float3 e = table_lerp(etab, fmaf(eB, t, eA));
           v.x = fmaf(th.gf[0], e.x, v.x);
           v.y = fmaf(th.gf[1], e.y, v.y);
           v.z = fmaf(th.gf[2], e.z, v.z);
         }
-        // l += x1 * v (x1 = 1 unless order 2 without ground term).
+        // l += x1 * v (with a ground term, x1 is in v).
         if (sgn == 0) {
-          l0 = kOrder2 && !kGround ? x1 * v.x : v.x;
-          l1 = kOrder2 && !kGround ? x1 * v.y : v.y;
-          l2 = kOrder2 && !kGround ? x1 * v.z : v.z;
-        } else if (kOrder2 && !kGround) {
+          l0 = kGround ? v.x : x1 * v.x;
+          l1 = kGround ? v.y : x1 * v.y;
+          l2 = kGround ? v.z : x1 * v.z;
+        } else if (!kGround) {
           l0 = fmaf(x1, v.x, l0);
           l1 = fmaf(x1, v.y, l1);
           l2 = fmaf(x1, v.z, l2);
@@ -611,7 +529,7 @@ template <int kChunk, int kB>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(5))) void
 k_scattering_density(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
-    int njobs, int order) {
+    int njobs) {
   extern __shared__ float4 lds[];
   __shared__ SdTheta th[kTheta];
   __shared__ int s_y0[kTheta], s_y1[kTheta];
@@ -638,13 +556,12 @@ k_scattering_density(
   const int im = pl % G, rest = pl / G;
   const int k = rest % J.nr, imus = (rest / J.nr) * G + im;
   const int W = nnu * nmus;
-  const bool two = order == 2;
   // Per theta a table of NU + 1 entries (table_lerp); then the
   // ground-irradiance table of E_W + 1 entries.
   const int stride = 2 * (nnu + 1);
   float4* tab_a = lds;
   float4* tab_b = lds + kTheta * stride;
-  float4* etab = lds + (two ? 2 : 1) * kTheta * stride;
+  float4* etab = lds + 2 * kTheta * stride;
   const int tid = threadIdx.x;
 
   double r, rho;
@@ -682,8 +599,8 @@ k_scattering_density(
   }
   __syncthreads();
 
-  // Per-theta nu tables of the order-(n-1) scattering at (r, mu_s), mu rows
-  // blended, times d_omega (and the phase-function constants for order 1).
+  // Per-theta nu tables of the single scattering at (r, mu_s), mu rows
+  // blended, times d_omega and the phase-function constants.
   const float kR = static_cast<float>(3.0 / (16.0 * kPi));
   const double gd = J.g;
   const float kM = static_cast<float>(3.0 / (8.0 * kPi) * (1.0 - gd * gd) / (2.0 + gd * gd));
@@ -694,7 +611,7 @@ k_scattering_density(
     const int c0 = n * nmus + imus;
     const int c1 = (n + 1 < nnu ? n + 1 : n) * nmus + imus;
     const float wy = s_wy[l], wy0 = 1.0f - wy;
-    const float fa = s_dw[l] * (two ? kR : 1.0f);
+    const float fa = s_dw[l] * kR;
     const float4* src = J.dR;
     float4 a0 = gload(src, r0 + c0), a1 = gload(src, r1 + c0);
     float4 b0 = gload(src, r0 + c1), b1 = gload(src, r1 + c1);
@@ -705,21 +622,19 @@ k_scattering_density(
     float4* ta = tab_a + l * stride;
     put_entry(ta, n + 1, v, vn);
     if (n == 0) put_entry(ta, 0, v, v);
-    if (two) {
-      const float fb = s_dw[l] * kM;
-      src = J.dM;
-      a0 = gload(src, r0 + c0);
-      a1 = gload(src, r1 + c0);
-      b0 = gload(src, r0 + c1);
-      b1 = gload(src, r1 + c1);
-      v = make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
-                      (wy0 * a0.z + wy * a1.z) * fb);
-      vn = make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
-                       (wy0 * b0.z + wy * b1.z) * fb);
-      float4* tb = tab_b + l * stride;
-      put_entry(tb, n + 1, v, vn);
-      if (n == 0) put_entry(tb, 0, v, v);
-    }
+    const float fb = s_dw[l] * kM;
+    src = J.dM;
+    a0 = gload(src, r0 + c0);
+    a1 = gload(src, r1 + c0);
+    b0 = gload(src, r0 + c1);
+    b1 = gload(src, r1 + c1);
+    v = make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
+                    (wy0 * a0.z + wy * a1.z) * fb);
+    vn = make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
+                     (wy0 * b0.z + wy * b1.z) * fb);
+    float4* tb = tab_b + l * stride;
+    put_entry(tb, n + 1, v, vn);
+    if (n == 0) put_entry(tb, 0, v, v);
   }
   // Row 0 of delta irradiance (r = rb): the ground-irradiance lookup of the
   // reference at bottom_radius reads exactly this row.
@@ -782,21 +697,12 @@ k_scattering_density(
     const float4* ta = tab_a + l * stride;
     const float4* tb = tab_b + l * stride;
     const bool g = __builtin_amdgcn_readfirstlane(t.ground) != 0;
-    if (two) {
-      if (g)
-        sd_theta<kChunk, true, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM,
-                             t, acc);
-      else
-        sd_theta<kChunk, true, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR,
-                              cM, t, acc);
-    } else {
-      if (g)
-        sd_theta<kChunk, false, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR,
-                              cM, t, acc);
-      else
-        sd_theta<kChunk, false, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR,
-                               cM, t, acc);
-    }
+    if (g)
+      sd_theta<kChunk, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+                             acc);
+    else
+      sd_theta<kChunk, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+                              acc);
   }
 #pragma unroll
   for (int jn = 0; jn < kChunk; ++jn) {
@@ -1639,25 +1545,24 @@ hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s) {
   return hipGetLastError();
 }
 template <int kChunk, int kB>
-void launch_sd_tile(const PassLaunch& p, int order, size_t lds, hipStream_t s) {
+void launch_sd_tile(const PassLaunch& p, size_t lds, hipStream_t s) {
   hipLaunchKernelGGL((k_scattering_density<kChunk, kB>), dim3(p.total_blocks), dim3(kB), lds,
-                     s, p.jobs, p.first_block, p.njobs, order);
+                     s, p.jobs, p.first_block, p.njobs);
 }
 
-hipError_t launch_scattering_density(const PassLaunch& p, int order,
-                                     hipStream_t s) {
+hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s) {
   // Tables of NU + 1 and E_W + 1 entries of two float4 (table_lerp).
   const size_t lds = sizeof(float4) *
-                     (static_cast<size_t>((order == 2 ? 4 : 2) * kTheta * (p.max_nnu + 1)) +
+                     (static_cast<size_t>(4 * kTheta * (p.max_nnu + 1)) +
                       2 * static_cast<size_t>(p.max_ew + 1));
   static_assert(kSdTiles == 6, "one case per tile shape");
   switch (p.tile) {
-    case 0: launch_sd_tile<kSdTile[0].chunk, kSdTile[0].block>(p, order, lds, s); break;
-    case 1: launch_sd_tile<kSdTile[1].chunk, kSdTile[1].block>(p, order, lds, s); break;
-    case 2: launch_sd_tile<kSdTile[2].chunk, kSdTile[2].block>(p, order, lds, s); break;
-    case 3: launch_sd_tile<kSdTile[3].chunk, kSdTile[3].block>(p, order, lds, s); break;
-    case 4: launch_sd_tile<kSdTile[4].chunk, kSdTile[4].block>(p, order, lds, s); break;
-    case 5: launch_sd_tile<kSdTile[5].chunk, kSdTile[5].block>(p, order, lds, s); break;
+    case 0: launch_sd_tile<kSdTile[0].chunk, kSdTile[0].block>(p, lds, s); break;
+    case 1: launch_sd_tile<kSdTile[1].chunk, kSdTile[1].block>(p, lds, s); break;
+    case 2: launch_sd_tile<kSdTile[2].chunk, kSdTile[2].block>(p, lds, s); break;
+    case 3: launch_sd_tile<kSdTile[3].chunk, kSdTile[3].block>(p, lds, s); break;
+    case 4: launch_sd_tile<kSdTile[4].chunk, kSdTile[4].block>(p, lds, s); break;
+    case 5: launch_sd_tile<kSdTile[5].chunk, kSdTile[5].block>(p, lds, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

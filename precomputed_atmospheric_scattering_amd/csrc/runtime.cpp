@@ -181,6 +181,7 @@ int pass_blocks(Pass p, const atmo::Job& j) {
     case kE0: return atmo::blocks_direct_irradiance(j);
     case kSS: return atmo::blocks_single_scattering(j);
     case kSD: return atmo::blocks_scattering_density(j);
+    case kSA: return atmo::blocks_density_arcs(j);
     case kII: return atmo::blocks_indirect_irradiance(j);
     case kMS: return atmo::blocks_multiple_scattering(j);
     case kHalf: return atmo::blocks_half_conversion(j);
@@ -360,6 +361,7 @@ void fill_job_luts(atmo_model* m, atmo::Job* j, int k) {
                                 (m->spec.half_precision ? sizeof(uint2) : sizeof(float3))
                : nullptr;
   j->niter = m->iters;
+  j->it = k >= 0 ? k : 0;
   j->OD = m->OD;  // every job of the model, the final transmittance's too
   set_sizes(j, m->sizes);
   j->combined = m->spec.combined ? 1 : 0;
@@ -408,13 +410,12 @@ atmo_status upload_jobs(atmo_model* m, unsigned orders, hipStream_t stream) {
   ATMO_HIP(hipMemcpyAsync(m->d_jobs, m->jobs.data(),
                           m->jobs.size() * sizeof(atmo::Job),
                           hipMemcpyHostToDevice, stream));
-  // Block prefixes of the model's launches (they follow the tiles): every
-  // job has the same sizes, so pass p's prefix over the iterations is
-  // {0, b, 2b, ...} with b = pass_blocks(p, job).
+  // Block prefixes of the model's launches (they follow the tiles).
   m->first_block_host.assign(kPasses * (iters + 1), 0);
   for (int p = 0; p < kPasses; ++p) {
-    const int b = pass_blocks(static_cast<Pass>(p), m->jobs[0]);
-    for (int i = 0; i <= iters; ++i) m->first_block_host[p * (iters + 1) + i] = i * b;
+    int* const fb = &m->first_block_host[p * (iters + 1)];
+    for (int i = 0; i < iters; ++i)
+      fb[i + 1] = fb[i] + pass_blocks(static_cast<Pass>(p), m->jobs[i]);
   }
   ATMO_HIP(hipMemcpyAsync(m->d_first_block, m->first_block_host.data(),
                           m->first_block_host.size() * sizeof(int), hipMemcpyHostToDevice,
@@ -437,6 +438,10 @@ atmo::PassLaunch model_launch(const atmo_model* m, int first_job, int njobs, Pas
   l.kinds = accumulates_fp64(m->spec) ? atmo::kJobsAcc64 : atmo::kJobsF32;
   l.dj_kinds = m->spec.half_precision ? atmo::kDjRgb21 : atmo::kDjF32;
   const atmo::Job& j = m->jobs[first_job];
+  l.arc_kinds = 0;
+  for (int i = 0; i < njobs; i += atmo::kArcIters)
+    l.arc_kinds |= atmo::arc_kind(m->jobs[first_job + i]);
+  l.arc_lds = atmo::arc_lds(j);
   l.tile = p == kSD ? j.sd_tile : (p == kMS ? j.ms_tile : 0);
   return l;
 }
@@ -512,7 +517,8 @@ atmo_status enqueue_precompute(atmo_model* m, unsigned orders, LaunchTimer& t) {
   for (unsigned order = 2; order <= orders; ++order) {
     const int o = static_cast<int>(order);
     ATMO_TRY(t.run(kSD, o, "scattering density", [&] {
-      return atmo::launch_scattering_density(model_launch(m, 0, n, kSD), o, s);
+      return order == 2 ? atmo::launch_scattering_density(model_launch(m, 0, n, kSD), s)
+                        : atmo::launch_density_arcs(model_launch(m, 0, n, kSA), s);
     }));
     ATMO_TRY(t.run(kII, o - 1, "indirect irradiance", [&] {
       return atmo::launch_indirect_irradiance(model_launch(m, 0, n, kII), o - 1, s);
@@ -1346,6 +1352,8 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     l.max_lds_w = 0;
     l.kinds = 0;
     l.dj_kinds = 0;
+    l.arc_kinds = 0;
+    l.arc_lds = 0;
     int total = 0;
     for (const auto& mj : sel) {
       const atmo::Job& j = models[mj.first]->jobs[mj.second];
@@ -1360,12 +1368,14 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
         l.max_lds_w = std::max(l.max_lds_w, j.nnu * j.nmus);
       l.kinds |= j.acc64 ? atmo::kJobsAcc64 : atmo::kJobsF32;
       l.dj_kinds |= j.half_luts ? atmo::kDjRgb21 : atmo::kDjF32;
+      if (j.it % atmo::kArcIters == 0) l.arc_kinds |= atmo::arc_kind(j);
+      l.arc_lds = std::max(l.arc_lds, atmo::arc_lds(j));
     }
     plan->first_block.push_back(total);
     l.total_blocks = total;
     plan->levels.push_back(l);
   };
-  // Scattering density and multiple scattering: one launch per tile shape
+  // Scattering density of order 2 and multiple scattering: one launch per tile shape
   // among the jobs (each kernel instance has one shape).
   auto add_level = [&](Pass p, int order, const std::vector<std::pair<int, int>>& sel) {
     if (p != kSD && p != kMS) {
@@ -1402,7 +1412,7 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     std::vector<std::pair<int, int>> on;
     for (const auto& mj : sel)
       if (orders[mj.first] >= n) on.push_back(mj);
-    add_level(kSD, static_cast<int>(n), on);
+    add_level(n == 2 ? kSD : kSA, static_cast<int>(n), on);
     add_level(kII, static_cast<int>(n) - 1, on);
     add_level(kMS, 0, on);
   }
@@ -1456,13 +1466,16 @@ atmo_status launch_level(const Level& l, const atmo::Job* d_jobs, const int* d_f
   pl.max_lds_w = l.max_lds_w;
   pl.kinds = l.kinds;
   pl.dj_kinds = l.dj_kinds;
+  pl.arc_kinds = l.arc_kinds;
+  pl.arc_lds = l.arc_lds;
   pl.tile = l.tile;
   hipError_t e = hipSuccess;
   switch (l.pass) {
     case kT: e = atmo::launch_transmittance(pl, s); break;
     case kE0: e = atmo::launch_direct_irradiance(pl, s); break;
     case kSS: e = atmo::launch_single_scattering(pl, s); break;
-    case kSD: e = atmo::launch_scattering_density(pl, l.order, s); break;
+    case kSD: e = atmo::launch_scattering_density(pl, s); break;
+    case kSA: e = atmo::launch_density_arcs(pl, s); break;
     case kII: e = atmo::launch_indirect_irradiance(pl, l.order, s); break;
     case kMS: e = atmo::launch_multiple_scattering(pl, s); break;
     case kClear: e = atmo::launch_clear_max(pl, s); break;

@@ -37,16 +37,19 @@ struct Sizes {
 };
 
 
-enum Pass { kT = 0, kE0, kSS, kSD, kII, kMS, kAcc, kHalf, kClear, kPack, kOD, kPasses };
+// kSD: scattering density of order 2; kSA: of the orders >= 3.
+enum Pass { kT = 0, kE0, kSS, kSD, kII, kMS, kAcc, kHalf, kClear, kPack, kOD, kSA, kPasses };
 
 
-// One launch of a batched pass sequence: pass kind, order argument, and the
-// segment of the plan's job and block-prefix arrays it uses.
+// One launch of a batched pass sequence: pass kind, order argument (SD and
+// SA: the order computed; II: the order read), and the segment of the plan's
+// job and block-prefix arrays it uses.
 struct Level {
   Pass pass;
-  int order;  // SD: order computed; II: order read; others unused
+  int order;
   int job_offset, njobs, fb_offset, total_blocks, max_nnu, max_ew, max_w, min_w, max_lds_w,
-      kinds, dj_kinds;
+      kinds, dj_kinds, arc_kinds;
+  size_t arc_lds;
   int tile;   // SD and MS: the tile shape shared by the level's jobs
 };
 
