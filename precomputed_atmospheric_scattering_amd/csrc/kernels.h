@@ -24,6 +24,7 @@ struct PassLaunch {
   int tile;     // tile shape of the jobs (scattering density, multiple
                 // scattering): every job of a launch has the same one
   int dj_kinds;  // kDjF32 | kDjRgb21: the delta J formats of the jobs
+  int sd_kinds;    // 1 << sd_split of the jobs, or-ed
   int arc_kinds;   // arc_kind of the jobs, or-ed
   size_t arc_lds;  // largest arc_lds of the jobs
 };
@@ -59,6 +60,35 @@ constexpr SdTile kSdTile[kSdTiles] = {{4, 256}, {2, 256}, {1, 256},
 // a LUT beyond the caches 4 times instead of 8.
 ATMO_HD int sd_default_tile(int nmu, int nnu) {
   return nmu * ((nnu + 3) / 4) <= 256 ? 3 : 0;
+}
+
+// Grids too small to fill the GPU at 4 outputs per thread: several threads
+// share an output, each summing some of the zenith angles, whatever the tile
+// shape. A job takes the first of these whose 'texels' it does not exceed (of
+// all its model's iterations), or none. Measured on MI355X (ms, 3 wavelengths
+// unless given; the shape of sd_default_tile in the first column):
+//   texels               1 part   4     8     16
+//   8192                  .287    -     -    .021
+//   32768                 .244  .096  .057   .032
+//   65536                 .243    -     -    .058
+//   131072                .268  .101  .078   .108
+//   262144                .274  .134  .137   .204
+//   524288                .334  .240  .248   .394
+//   1048576               .491  .423  .484   .774
+//   3 x 391230 (9 wl)     .63   .573  .664
+//   5 x 262144 (15 wl)    .518  .543  .600   .973
+struct SdSplit {
+  int chunk, block, parts, texels;
+};
+constexpr int kSdSplits = 3;
+constexpr SdSplit kSdSplit[kSdSplits] = {
+    {1, 1024, 16, 1 << 16}, {4, 512, 8, 1 << 18}, {4, 256, 4, 1250000}};
+// The job's index into kSdSplit, or kSdSplits.
+ATMO_HD int sd_split(const Job& j) {
+  const int64_t n = static_cast<int64_t>(j.nr) * j.nmu * j.nmus * j.nnu * j.niter;
+  int i = 0;
+  while (i < kSdSplits && n > kSdSplit[i].texels) ++i;
+  return i;
 }
 
 // Scattering density of orders >= 3 (density_arcs.h): a block of 8 waves

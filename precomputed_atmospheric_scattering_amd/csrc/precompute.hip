@@ -525,7 +525,10 @@ __device__ __forceinline__ void sd_theta(
 // Five waves per SIMD: the 4-output shapes then fit 96 VGPRs (101 unbounded,
 // four waves), and the pass, which issues a VALU instruction in about 90% of
 // the SIMD cycles, runs 2-3% faster on MI355X.
-template <int kChunk, int kB>
+//
+// kParts: threads that share an output, each summing kTheta / kParts of the
+// zenith angles (kSdSplit; 1 for the jobs that take none of it).
+template <int kChunk, int kB, int kParts>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(5))) void
 k_scattering_density(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
@@ -537,10 +540,13 @@ k_scattering_density(
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
   const int lb = blockIdx.x - first_block[ji];
+  const int split = sd_split(J);
+  if ((split == kSdSplits ? 1 : kSdSplit[split].parts) != kParts) return;
   const int nnu = J.nnu, nmus = J.nmus, nmu = J.nmu;
   const int nch = (nnu + kChunk - 1) / kChunk;
-  const int plane = nmu * nch;  // threads per (r, mu_s) plane
-  const int tiles = (plane + kB - 1) / kB;
+  const int plane = nmu * nch;  // threads per (r, mu_s) plane and part
+  constexpr int kOuts = kB / kParts;
+  const int tiles = (plane + kOuts - 1) / kOuts;
   // The blocks of neighbouring mu_s columns of a layer write the same cache
   // lines of delta J (a plane's texels are W texels apart). The block order
   // walks groups of G consecutive mu_s columns (G = the largest power of two
@@ -646,9 +652,10 @@ k_scattering_density(
   }
   __syncthreads();
 
-  const int flat = tile * kB + tid;
-  if (flat >= plane) return;
-  const int ch = flat % nch, y = flat / nch;
+  const int part = tid / kOuts;
+  const int flat = tile * kOuts + (kParts > 1 ? tid % kOuts : tid);
+  if (kParts == 1 && flat >= plane) return;
+  const int ch = flat % nch, y = min(flat / nch, nmu - 1);
   double mu;
   bool ground_unused;
   s_row_mu(J, y, r, rho, &mu, &ground_unused);
@@ -685,7 +692,8 @@ k_scattering_density(
   float acc[kChunk][3];
 #pragma unroll
   for (int jn = 0; jn < kChunk; ++jn) acc[jn][0] = acc[jn][1] = acc[jn][2] = 0.0f;
-  for (int l = 0; l < kTheta; ++l) {
+  constexpr int kAngles = kTheta / kParts;
+  for (int l = part * kAngles; l < (part + 1) * kAngles; ++l) {
     const SdTheta t = th[l];
     const float A = fmus * t.cos_t, P = fmu * t.cos_t, Q = fwx * t.sin_t;
     float Bv[kChunk], Cv[kChunk];
@@ -703,6 +711,23 @@ k_scattering_density(
     else
       sd_theta<kChunk, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
                               acc);
+  }
+  if (kParts > 1) {
+    // The parts of an output, in place of the tables, summed by the threads
+    // of the first.
+    float* const sums = reinterpret_cast<float*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int jn = 0; jn < kChunk; ++jn)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) sums[(jn * 3 + c) * kB + tid] = acc[jn][c];
+    __syncthreads();
+    if (part != 0 || flat >= plane) return;
+    for (int q = 1; q < kParts; ++q)
+#pragma unroll
+      for (int jn = 0; jn < kChunk; ++jn)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) acc[jn][c] += sums[(jn * 3 + c) * kB + q * kOuts + tid];
   }
 #pragma unroll
   for (int jn = 0; jn < kChunk; ++jn) {
@@ -1483,8 +1508,12 @@ int blocks_single_scattering(const Job& j) {
 }
 int blocks_scattering_density(const Job& j) {
   const SdTile t = kSdTile[j.sd_tile];
-  const int plane = j.nmu * ((j.nnu + t.chunk - 1) / t.chunk);
-  return ((plane + t.block - 1) / t.block) * j.nmus * j.nr;
+  const int split = sd_split(j);
+  const int chunk = split < kSdSplits ? kSdSplit[split].chunk : t.chunk;
+  const int outs =
+      split < kSdSplits ? kSdSplit[split].block / kSdSplit[split].parts : t.block;
+  const int plane = j.nmu * ((j.nnu + chunk - 1) / chunk);
+  return ((plane + outs - 1) / outs) * j.nmus * j.nr;
 }
 int blocks_indirect_irradiance(const Job& j) { return j.ew * j.eh; }
 int blocks_multiple_scattering(const Job& j) {
@@ -1546,8 +1575,19 @@ hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s) {
 }
 template <int kChunk, int kB>
 void launch_sd_tile(const PassLaunch& p, size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL((k_scattering_density<kChunk, kB>), dim3(p.total_blocks), dim3(kB), lds,
+  hipLaunchKernelGGL((k_scattering_density<kChunk, kB, 1>), dim3(p.total_blocks), dim3(kB), lds,
                      s, p.jobs, p.first_block, p.njobs);
+}
+
+template <int kSplit>
+void launch_sd_split(const PassLaunch& p, size_t lds, hipStream_t s) {
+  constexpr SdSplit t = kSdSplit[kSplit];
+  static_assert(t.block / t.parts == 64, "a wave's outputs share their zenith angles");
+  const size_t sums = sizeof(float) * 3 * t.chunk * t.block;
+  if (p.sd_kinds & (1 << kSplit))
+    hipLaunchKernelGGL((k_scattering_density<t.chunk, t.block, t.parts>), dim3(p.total_blocks),
+                       dim3(t.block), lds > sums ? lds : sums, s, p.jobs, p.first_block,
+                       p.njobs);
 }
 
 hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s) {
@@ -1556,6 +1596,11 @@ hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s) {
                      (static_cast<size_t>(4 * kTheta * (p.max_nnu + 1)) +
                       2 * static_cast<size_t>(p.max_ew + 1));
   static_assert(kSdTiles == 6, "one case per tile shape");
+  static_assert(kSdSplits == 3, "one launch per split");
+  launch_sd_split<0>(p, lds, s);
+  launch_sd_split<1>(p, lds, s);
+  launch_sd_split<2>(p, lds, s);
+  if ((p.sd_kinds & (1 << kSdSplits)) == 0) return hipGetLastError();
   switch (p.tile) {
     case 0: launch_sd_tile<kSdTile[0].chunk, kSdTile[0].block>(p, lds, s); break;
     case 1: launch_sd_tile<kSdTile[1].chunk, kSdTile[1].block>(p, lds, s); break;

@@ -438,6 +438,7 @@ atmo::PassLaunch model_launch(const atmo_model* m, int first_job, int njobs, Pas
   l.kinds = accumulates_fp64(m->spec) ? atmo::kJobsAcc64 : atmo::kJobsF32;
   l.dj_kinds = m->spec.half_precision ? atmo::kDjRgb21 : atmo::kDjF32;
   const atmo::Job& j = m->jobs[first_job];
+  l.sd_kinds = 1 << atmo::sd_split(j);
   l.arc_kinds = 0;
   for (int i = 0; i < njobs; i += atmo::kArcIters)
     l.arc_kinds |= atmo::arc_kind(m->jobs[first_job + i]);
@@ -1352,7 +1353,7 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     l.max_lds_w = 0;
     l.kinds = 0;
     l.dj_kinds = 0;
-    l.arc_kinds = 0;
+    l.sd_kinds = l.arc_kinds = 0;
     l.arc_lds = 0;
     int total = 0;
     for (const auto& mj : sel) {
@@ -1368,6 +1369,7 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
         l.max_lds_w = std::max(l.max_lds_w, j.nnu * j.nmus);
       l.kinds |= j.acc64 ? atmo::kJobsAcc64 : atmo::kJobsF32;
       l.dj_kinds |= j.half_luts ? atmo::kDjRgb21 : atmo::kDjF32;
+      l.sd_kinds |= 1 << atmo::sd_split(j);
       if (j.it % atmo::kArcIters == 0) l.arc_kinds |= atmo::arc_kind(j);
       l.arc_lds = std::max(l.arc_lds, atmo::arc_lds(j));
     }
@@ -1466,6 +1468,7 @@ atmo_status launch_level(const Level& l, const atmo::Job* d_jobs, const int* d_f
   pl.max_lds_w = l.max_lds_w;
   pl.kinds = l.kinds;
   pl.dj_kinds = l.dj_kinds;
+  pl.sd_kinds = l.sd_kinds;
   pl.arc_kinds = l.arc_kinds;
   pl.arc_lds = l.arc_lds;
   pl.tile = l.tile;
