@@ -293,7 +293,10 @@ atmo_status atmo_model_get_lut(const atmo_model* model, atmo_lut_id id,
 atmo_status atmo_model_copy_lut(const atmo_model* model, atmo_lut_id id,
                                 float* host_rgba);
 /* Device bytes held by the model's result LUTs, and the peak extra bytes
- * Init allocates for its temporaries. */
+ * Init allocates for its temporaries. Between calls of atmo_model_init the
+ * library keeps the block of the last one on a device (at most 1 GiB) for the
+ * next; it is freed with the last model, or when an allocation of the library
+ * finds no memory. */
 atmo_status atmo_model_footprint(const atmo_model* model, size_t* resident,
                                  size_t* init_scratch);
 

@@ -180,8 +180,8 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
   ATMO_TRY(atmo_model_init_batch(models.data(), orders.data(), k, s));
 
   DeviceArrays d;
-  TUNE_HIP(hipMalloc(&d.jobs, k * sizeof(atmo::Job)));
-  TUNE_HIP(hipMalloc(&d.first_block, (k + 1) * sizeof(int)));
+  TUNE_HIP(device_malloc(&d.jobs, k * sizeof(atmo::Job)));
+  TUNE_HIP(device_malloc(&d.first_block, (k + 1) * sizeof(int)));
   TUNE_HIP(hipEventCreate(&d.start));
   TUNE_HIP(hipEventCreate(&d.stop));
   const int w = z.nnu * z.nmus;

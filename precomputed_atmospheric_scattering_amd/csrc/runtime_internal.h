@@ -60,6 +60,22 @@ struct LevelPlan {
   std::vector<Level> levels;
 };
 
+// Counts the models alive: with the last one the block of temporaries kept
+// between calls of Init is freed.
+struct LiveModel {
+  LiveModel();
+  ~LiveModel();
+  LiveModel(const LiveModel&) = delete;
+};
+// Frees the blocks kept between calls of Init; whether there were any.
+bool trim_temporaries_pool();
+// hipMalloc, which frees those blocks if memory is out.
+hipError_t device_malloc(void** p, size_t bytes);
+template <class T>
+hipError_t device_malloc(T** p, size_t bytes) {
+  return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
+
 }  // namespace atmo_rt
 
 // A model: parameters, LUTs, temporaries, job tables.
@@ -68,6 +84,7 @@ struct atmo_model {
   using Spec = atmo_rt::Spec;
   using Sizes = atmo_rt::Sizes;
   static constexpr int kPasses = atmo_rt::kPasses;
+  atmo_rt::LiveModel live;
   Spec spec;
   Sizes sizes;
   int device = 0;
@@ -85,6 +102,8 @@ struct atmo_model {
   // transmittance and irradiance accumulators at T_it and E_it. dE, dR, dM,
   // dJ point at the last iteration's copies (the retained intermediates).
   char* temp_block = nullptr;
+  size_t temp_bytes = 0;  // of temp_block
+  int temp_device = 0;
   float4 *T_it = nullptr, *E_it = nullptr;
   float4 *dE_it = nullptr, *dR_it = nullptr, *dM_it = nullptr;
   float4 *dE = nullptr, *dR = nullptr, *dM = nullptr;

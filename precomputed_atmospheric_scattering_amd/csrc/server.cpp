@@ -302,7 +302,7 @@ struct atmo_server {
     if (*cap >= need) return true;
     size_t n = std::max(need, *cap * 2);
     void* p = nullptr;
-    if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) return false;
+    if (device_malloc(&p, n * sizeof(T)) != hipSuccess) return false;
     if (*ptr != nullptr) graveyard_ptrs.push_back(*ptr);
     *ptr = static_cast<T*>(p);
     *cap = n;
@@ -387,7 +387,7 @@ struct atmo_server {
       s.arena = nullptr;
       s.arena_bytes = 0;
       void* p = nullptr;
-      if (hipMalloc(&p, scratch) != hipSuccess) {
+      if (device_malloc(&p, scratch) != hipSuccess) {
         fail_batch(batch, made, ATMO_ERROR_OUT_OF_MEMORY);
         return;
       }
@@ -594,6 +594,7 @@ atmo_status atmo_server_create(const atmo_server_config* config, atmo_server** o
   if (s->cfg.lookup_streams <= 0) s->cfg.lookup_streams = 2;
   if (hipGetDevice(&s->device) != hipSuccess)
     return fail(ATMO_ERROR_DEVICE, "hipGetDevice failed");
+  trim_temporaries_pool();  // counted as free
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
     return fail(ATMO_ERROR_DEVICE, "hipMemGetInfo failed");
