@@ -212,6 +212,8 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     pl.max_lds_w = w <= atmo::kMsMaxRow ? w : 0;
     pl.kinds = atmo::kJobsF32;
     pl.dj_kinds = atmo::kDjF32;
+    pl.ss_kinds = 0;
+    pl.ss_lds = 0;
     pl.sd_kinds = 1 << atmo::sd_split(js[0]);
     pl.arc_kinds = 0;
     pl.arc_lds = 0;

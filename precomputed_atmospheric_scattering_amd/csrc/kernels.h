@@ -24,6 +24,8 @@ struct PassLaunch {
   int tile;     // tile shape of the jobs (scattering density, multiple
                 // scattering): every job of a launch has the same one
   int dj_kinds;  // kDjF32 | kDjRgb21: the delta J formats of the jobs
+  int ss_kinds;    // ss_kind of the jobs, or-ed
+  size_t ss_lds;   // largest ss_lds of the jobs
   int sd_kinds;    // 1 << sd_split of the jobs, or-ed
   int arc_kinds;   // arc_kind of the jobs, or-ed
   size_t arc_lds;  // largest arc_lds of the jobs
@@ -89,6 +91,51 @@ ATMO_HD int sd_split(const Job& j) {
   int i = 0;
   while (i < kSdSplits && n > kSdSplit[i].texels) ++i;
   return i;
+}
+
+// Single scattering: blocks of 'block' texels of a packed row, for 'nit'
+// iterations of a model, ss_staged of them with the blended transmittance rows
+// of a sample in LDS (TW up to 4096: 98 KB at most for one). The figures are
+// at k_single_scattering.
+constexpr int kSsIters = 5;
+constexpr int kSsRowBytes = 64 << 10;  // at most, if iterations share a block
+constexpr int kSsGroupBlocks = 512;
+constexpr ATMO_HD int ss_staged(int nit, int block) {
+  return block < kBlock ? 0 : (nit < 3 ? 1 : 2);
+}
+template <bool kF64>
+constexpr int kSsBuffers = kF64 ? 1 : 2;
+ATMO_HD size_t ss_row_bytes(const Job& j, int nit, int block) {
+  const size_t texels = static_cast<size_t>(ss_staged(nit, block)) * j.tw * 3;
+  return texels * (j.acc64 ? kSsBuffers<true> * sizeof(double)
+                           : kSsBuffers<false> * sizeof(float));
+}
+struct SsTiling {
+  int block;
+  int nit;  // 0: the job is served by the blocks of an earlier iteration
+  ATMO_HD explicit SsTiling(const Job& j) {
+    const int w = j.nnu * j.nmus, most = j.niter < kSsIters ? j.niter : kSsIters;
+    block = w > kBlock ? 2 * kBlock : (w > 64 ? kBlock : 64);
+    const int64_t blocks = static_cast<int64_t>(j.nr) * j.nmu * ((w + block - 1) / block);
+    nit = 1;
+    // Iterations share a block once that leaves two blocks per CU.
+    if (most > 1 && ss_row_bytes(j, most, block) <= kSsRowBytes && blocks >= kSsGroupBlocks) {
+      const int left = j.niter - j.it;
+      nit = j.it % kSsIters != 0 ? 0 : (left < kSsIters ? left : kSsIters);
+    }
+  }
+};
+// PassLaunch::ss_kinds.
+constexpr int ss_kind(bool f64, int nit, int block) {
+  return 1 << ((f64 ? nit : 0) + (block > kBlock ? 2 : (block == kBlock ? 1 : 0)) * (kSsIters + 1));
+}
+ATMO_HD int ss_kind(const Job& j) {
+  const SsTiling t(j);
+  return t.nit == 0 ? 0 : ss_kind(j.acc64 != 0, t.nit, t.block);
+}
+inline size_t ss_lds(const Job& j) {
+  const SsTiling t(j);
+  return ss_row_bytes(j, t.nit, t.block);
 }
 
 // Scattering density of orders >= 3 (density_arcs.h): a block of 8 waves

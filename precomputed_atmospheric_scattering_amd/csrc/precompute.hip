@@ -130,8 +130,7 @@ __global__ __launch_bounds__(kBlock) void k_direct_irradiance(
 // Single scattering (functions.glsl:650-730, :933-945) and the output packing
 // of atmosphere/model.cc:142-157.
 //
-// A block covers up to 256 texels of one packed row (fixed r layer and mu
-// row). Along a row only mu_s and nu change, so every quantity of the 51
+// A block covers texels of one packed row (fixed r layer and mu row). Along a row only mu_s and nu change, so every quantity of the 51
 // ray-march samples that depends on (r, mu, d_i) alone - the view
 // transmittance, the densities, the transmittance-LUT row of the sample
 // radius - is computed once per block in FP64 and kept in LDS. Per texel and
@@ -154,68 +153,87 @@ __device__ __forceinline__ int split_coord(float t, float* frac) {
 // and the horizon term of every texel in FP64 in both.
 template <class Real>
 struct SsSample {
-  double d;        // distance along the view ray
-  double inv_r;    // 1 / r_d
   double rho;      // sqrt(r_d^2 - rb^2)
   Real r;          // r_d
   Real c;          // rt^2 - r_d^2
   Real dmin;       // rt - r_d
-  Real inv_range;  // 1 / (rho + H - dmin)
-  Real e;          // sin(theta_h) * sun angular radius
-  Real inv_span;   // 1 / (2 e)
+  Real per_column; // (TW - 1) / (rho + H - dmin)
+  Real per_disc;   // 1 / (2 r_d sin(theta_h) * sun angular radius)
   Real wy;
+  Real dr, dm;     // trapezoid weight * Rayleigh, Mie density
   int t0, t1;      // first texels of the transmittance LUT rows of r_d
-  Real fr[3];      // trapezoid weight * view transmittance * Rayleigh density
-  Real fm[3];      // same with the Mie density
 };
 
-// functions.glsl:402-421 at (r_d, mu_s_d): DistanceToTopAtmosphereBoundary
-// in the cancellation-free form, the LUT column coordinate, and the bilinear
-// transmittance lookup (functions.glsl:473-480).
-__device__ __forceinline__ void tsun_lookup(const Job& J, const SsSample<float>& S,
-                                            float mus, float o[3]) {
-  const float tt = S.r * mus;
-  const float sq = sqrt_f(fmaf(tt, tt, S.c));
-  const float dd = tt > 0.0f ? S.c * rcp_f(sq + tt) : sq - tt;
-  const float xm = (dd - S.dmin) * S.inv_range;
-  const float ut = clamp_index_coord(xm * static_cast<float>(J.tw - 1),
-                                     static_cast<float>(J.tw - 1));
-  float w;
-  const int i0 = split_coord(ut, &w);
-  const int i1 = min(i0 + 1, J.tw - 1);
-  const float4* __restrict__ T = J.T;
-  const uint32_t r0 = static_cast<uint32_t>(S.t0), r1 = static_cast<uint32_t>(S.t1);
-  const float4 a = gload32(T, r0 + i0), b = gload32(T, r0 + i1);
-  const float4 c = gload32(T, r1 + i0), d = gload32(T, r1 + i1);
-  const float wy1 = S.wy, wy0 = 1.0f - S.wy;
-  o[0] = fmaf(wy1, fmaf(w, d.x - c.x, c.x), wy0 * fmaf(w, b.x - a.x, a.x));
-  o[1] = fmaf(wy1, fmaf(w, d.y - c.y, c.y), wy0 * fmaf(w, b.y - a.y, a.y));
-  o[2] = fmaf(wy1, fmaf(w, d.z - c.z, c.z), wy0 * fmaf(w, b.z - a.z, a.z));
+// Sample i of the view ray (r, mu).
+template <class Real>
+__device__ void ss_sample(const Job& J, double r, double mu, int i, double dx,
+                          SsSample<Real>* out) {
+  SsSample<Real>& S = *out;
+  const double d = i * dx;
+  const double r_d = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
+  const double rho_d = safe_sqrt(r_d * r_d - J.rb * J.rb);
+  S.rho = rho_d;
+  S.r = static_cast<Real>(r_d);
+  S.c = static_cast<Real>(J.rt * J.rt - r_d * r_d);
+  S.dmin = static_cast<Real>(J.rt - r_d);
+  S.per_column = static_cast<Real>((J.tw - 1) / (rho_d + J.H - (J.rt - r_d)));
+  S.per_disc = static_cast<Real>(0.5 / (J.rb * J.sun_angular_radius));
+  const double ty = unit_to_texel(rho_d / J.H, J.th);
+  const Taps tt = axis_taps(ty, J.th);
+  S.t0 = tt.i0 * J.tw;
+  S.t1 = tt.i1 * J.tw;
+  // The exact weight in FP64 (Taps rounds it to float).
+  const double cy = fmin(fmax(ty, -1.0), static_cast<double>(J.th));
+  S.wy = sizeof(Real) == 8 ? static_cast<Real>(cy - floor(cy)) : static_cast<Real>(tt.w);
+  const double w = (i == 0 || i == kMarch - 1) ? 0.5 : 1.0;
+  S.dr = static_cast<Real>(w * profile_density(J.prof_r, r_d - J.rb));
+  S.dm = static_cast<Real>(w * profile_density(J.prof_m, r_d - J.rb));
 }
 
-// In FP64 the distance needs no cancellation-free form: sq - tt loses at most
+// Transmittance of the view ray up to distance d.
+__device__ __forceinline__ void ss_view(const Job& J, double r, double mu, double d,
+                                        bool ground, float (&tv)[3]) {
+  const float3 t = transmittance(J, J.T, r, mu, d, ground);
+  tv[0] = t.x;
+  tv[1] = t.y;
+  tv[2] = t.z;
+}
+__device__ __forceinline__ void ss_view(const Job& J, double r, double mu, double d,
+                                        bool ground, double (&tv)[3]) {
+  const D4 t = transmittance_d(J, J.T, r, mu, d, ground);
+  tv[0] = t.x;
+  tv[1] = t.y;
+  tv[2] = t.z;
+}
+
+// Column coordinate of the transmittance LUT (functions.glsl:402-421) at
+// r_d mu_s_d = t: DistanceToTopAtmosphereBoundary in the cancellation-free
+// form.
+__device__ __forceinline__ float ss_column(const Job& J, const SsSample<float>& S, float t) {
+  const float sq = sqrt_f(fmaf(t, t, S.c));
+  const float dd = t > 0.0f ? S.c * rcp_f(sq + t) : sq - t;
+  return clamp_index_coord((dd - S.dmin) * S.per_column, static_cast<float>(J.tw - 1));
+}
+// In FP64 the distance needs no cancellation-free form: sq - t loses at most
 // about 1e-16 sq = 6e-13 km, 1e-13 texel of the LUT coordinate, and saves a
 // division and a divergent branch per sample.
-__device__ __forceinline__ void tsun_lookup(const Job& J, const SsSample<double>& S,
-                                            double mus, double o[3]) {
-  const double tt = S.r * mus;
-  const double sq = sqrt(fma(tt, tt, S.c));
-  const double dd = sq - tt;
-  double ut = (dd - S.dmin) * S.inv_range * (J.tw - 1);
-  ut = fmin(fmax(ut, 0.0), static_cast<double>(J.tw - 1));
-  // ut >= 0: truncation is floor, and v_fract_f64 gives ut - floor(ut)
-  // exactly (as split_coord in FP32).
-  const double w = __builtin_amdgcn_fract(ut);
-  const int i0 = static_cast<int>(ut);
-  const int i1 = min(i0 + 1, J.tw - 1);
-  const float4* __restrict__ T = J.T;
-  const uint32_t r0 = static_cast<uint32_t>(S.t0), r1 = static_cast<uint32_t>(S.t1);
-  const float4 a = gload32(T, r0 + i0), b = gload32(T, r0 + i1);
-  const float4 c = gload32(T, r1 + i0), d = gload32(T, r1 + i1);
-  const double wy1 = S.wy, wy0 = 1.0 - S.wy;
-  o[0] = fma(wy1, fma(w, double(d.x) - c.x, double(c.x)), wy0 * fma(w, double(b.x) - a.x, double(a.x)));
-  o[1] = fma(wy1, fma(w, double(d.y) - c.y, double(c.y)), wy0 * fma(w, double(b.y) - a.y, double(a.y)));
-  o[2] = fma(wy1, fma(w, double(d.z) - c.z, double(c.z)), wy0 * fma(w, double(b.z) - a.z, double(a.z)));
+__device__ __forceinline__ double ss_column(const Job& J, const SsSample<double>& S, double t) {
+  const double ut = (sqrt(fma(t, t, S.c)) - t - S.dmin) * S.per_column;
+  return fmin(fmax(ut, 0.0), static_cast<double>(J.tw - 1));
+}
+
+// The sun seen from sample S, t = r_d mu_s_d: the visible part of its disc
+// (GetTransmittanceToSun, functions.glsl:473-480; r_d sin(theta_h) is the
+// bottom radius) and the transmittance column *u.
+template <class Real>
+__device__ __forceinline__ Real ss_sun(const Job& J, const SsSample<Real>& S, double t,
+                                       Real* u) {
+  // Clamps as max/min, 2 instructions each (the operands are finite; the
+  // ternary form, which also keeps NaNs, compiles to compares and selects).
+  const Real v = fmin(
+      fmax(fma(static_cast<Real>(t + S.rho), S.per_disc, Real(0.5)), Real(0)), Real(1));
+  *u = ss_column(J, S, fmin(fmax(static_cast<Real>(t), -S.r), S.r));
+  return v * v * fma(Real(-2), v, Real(3));
 }
 
 // The outputs of one single-scattering texel: the delta Rayleigh and Mie
@@ -248,34 +266,46 @@ __device__ __forceinline__ void ss_store(const Job& J, int64_t t_idx, double dx,
   if (!J.combined) gstore(J.SM, t_idx, make_float4(lm.x, lm.y, lm.z, 0.0f));
 }
 
-// Texels per thread of the single-scattering pass for packed rows of W
-// texels: 2 once a row fills two blocks (texels x and x + kBlock of a row
-// then share each sample's transmittance rows), else 1.
-__host__ __device__ inline int ss_texels_per_thread(int w) {
-  return w >= 4 * kBlock ? 4 : (w >= 2 * kBlock ? 2 : 1);
-}
-
+// A block covers up to kB texels of one packed row for kNit Precompute
+// iterations of a model: where along the view ray the sun is seen, and at
+// which transmittance texel, does not depend on the wavelength. The two
+// transmittance rows of a sample's radius are the same for all texels of the
+// packed row: for ss_staged of the iterations the block blends them, times the
+// view transmittance, into LDS, and a texel interpolates between two
+// neighbours there; for the others it gathers its four texels from memory
+// (16 bytes a lane, 16 L1 cycles each). With all of them gathered, and the
+// geometry found for each iteration, the pass issued vector instructions in 99%
+// of the cycles at the reference sizes with 79% of the L1's; with all staged
+// the LDS (FP64 rows, read at random) is what limits it. On MI355X, ms per Init
+// of one iteration per block all gathered | 5 iterations with 5, 4, 3, 2, 1, 0
+// staged:
+//   1.05M texels, 15 wavelengths   .80 | .77  .69  .65  .62  .68  .83
+//   16.8M, 15                      16.4 | 14.5 13.6 12.5 11.5 12.4 26
+// and of 3 iterations with 2, 1 staged .195, .207 (.39M texels; before .22). One
+// FP32 iteration, gathered | staged: .153 | .130 at 1.05M texels, 2.8 | 1.8 at
+// 16.8M. Rows of at most 64 texels are gathered by single waves: staged, 32
+// texels wide rows took .025 ms against .021 at 8192 texels.
 // kF64: the kernel serves the jobs with FP64 accumulators (illuminance
 // mode) and computes the sun-side lookups and the sums in FP64; otherwise it
-// serves the others. kTpt: texels per thread, ss_texels_per_thread(W) of the
-// job: texels x + k kBlock (k < kTpt) of one row, whose sun lookups read the
-// same two transmittance rows per sample, so a wave keeps kTpt times the
-// gathers in flight and the later texels often find their lines in L1. The
-// instances are launched over the same blocks when a launch holds several
-// kinds; each returns at once on the others' jobs.
-template <bool kF64, int kTpt>
-__global__ __launch_bounds__(kBlock) void k_single_scattering(
-    const Job* __restrict__ jobs, const int* __restrict__ first_block,
-    int njobs) {
+// serves the others. The instances are launched over the same blocks when a
+// launch holds several kinds; each returns at once on the others' jobs.
+template <bool kF64, int kNit, int kB>
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void
+k_single_scattering(
+    const Job* __restrict__ jobs, const int* __restrict__ first_block, int njobs) {
   using Real = typename std::conditional<kF64, double, float>::type;
+  // The blended rows of the iterations: kSsBuffers x [kNit][TW] RGB texels.
+  extern __shared__ float4 ss_lds[];
+  Real* const rows = reinterpret_cast<Real*>(ss_lds);
   __shared__ SsSample<Real> smp[kMarch];
+  __shared__ Real tv[kMarch][kNit][3];
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
-  if ((J.acc64 != 0) != kF64) return;
+  const SsTiling tl(J);
+  if ((J.acc64 != 0) != kF64 || tl.nit != kNit || tl.block != kB) return;
   const int W = J.nnu * J.nmus;
-  if (ss_texels_per_thread(W) != kTpt) return;
   const int lb = blockIdx.x - first_block[ji];
-  const int tiles = (W + kBlock * kTpt - 1) / (kBlock * kTpt);
+  const int tiles = (W + kB - 1) / kB;
   const int tile = lb % tiles;
   const int row = lb / tiles;  // z * nmu + y
   const int y = row % J.nmu, z = row / J.nmu;
@@ -286,101 +316,98 @@ __global__ __launch_bounds__(kBlock) void k_single_scattering(
   s_layer_r(J, z, &r, &rho);
   s_row_mu(J, y, r, rho, &mu, &ground);
   const double dx = dist_nearest(J, r, mu, ground) / (kMarch - 1);
-
-  if (tid < kMarch) {
-    SsSample<Real>& S = smp[tid];
-    const double d = tid * dx;
-    const double r_d = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
-    double tv[3];
-    if (kF64) {
-      const D4 t = transmittance_d(J, J.T, r, mu, d, ground);
-      tv[0] = t.x;
-      tv[1] = t.y;
-      tv[2] = t.z;
-    } else {
-      const float3 t = transmittance(J, J.T, r, mu, d, ground);
-      tv[0] = t.x;
-      tv[1] = t.y;
-      tv[2] = t.z;
-    }
-    const double rho_d = safe_sqrt(r_d * r_d - J.rb * J.rb);
-    S.d = d;
-    S.inv_r = 1.0 / r_d;
-    S.rho = rho_d;
-    S.r = static_cast<Real>(r_d);
-    S.c = static_cast<Real>(J.rt * J.rt - r_d * r_d);
-    S.dmin = static_cast<Real>(J.rt - r_d);
-    S.inv_range = static_cast<Real>(1.0 / (rho_d + J.H - (J.rt - r_d)));
-    const double e = J.rb / r_d * J.sun_angular_radius;
-    S.e = static_cast<Real>(e);
-    S.inv_span = static_cast<Real>(0.5 / e);
-    const double ty = unit_to_texel(rho_d / J.H, J.th);
-    const Taps tt = axis_taps(ty, J.th);
-    S.t0 = tt.i0 * J.tw;
-    S.t1 = tt.i1 * J.tw;
-    if (kF64) {
-      // The exact weight (Taps rounds it to float).
-      const double cy = fmin(fmax(ty, -1.0), static_cast<double>(J.th));
-      S.wy = static_cast<Real>(cy - floor(cy));
-    } else {
-      S.wy = static_cast<Real>(tt.w);
-    }
-    const double w = (tid == 0 || tid == kMarch - 1) ? 0.5 : 1.0;
-    const double dr = w * profile_density(J.prof_r, r_d - J.rb);
-    const double dm = w * profile_density(J.prof_m, r_d - J.rb);
-    for (int c = 0; c < 3; ++c) {
-      S.fr[c] = static_cast<Real>(dr * tv[c]);
-      S.fm[c] = static_cast<Real>(dm * tv[c]);
-    }
+  if (tid < kMarch) ss_sample(J, r, mu, tid, dx, &smp[tid]);
+  for (int e = tid; e < kMarch * kNit; e += kB) {
+    const int q = e / kMarch, s = e - q * kMarch;
+    ss_view((&J)[q], r, mu, s * dx, ground, tv[s][q]);
   }
+
+  const int x = tile * kB + tid;
+  const bool on = x < W;
+  const double mu_s = on ? s_col_mus(J, x % J.nmus) : 0.0;
+  const double nu = on ? s_slice_nu(J, x / J.nmus, mu, mu_s) : 0.0;
+  const double rmus = r * mu_s;
+  Real ar[kNit][3] = {}, am[kNit][3] = {};
+  const int tw = J.tw;
+  const float4* __restrict__ T[kNit];
+#pragma unroll
+  for (int k = 0; k < kNit; ++k) T[k] = (&J)[k].T;
+  constexpr int kStaged = ss_staged(kNit, kB);
+  constexpr bool kTwo = kSsBuffers<kF64> == 2;
+  float4 a[kStaged + 1], b[kStaged + 1];
+  auto fetch = [&](int s, int c) {
+#pragma unroll
+    for (int k = 0; k < kStaged; ++k) {
+      a[k] = gload32(T[k], static_cast<uint32_t>(smp[s].t0 + c));
+      b[k] = gload32(T[k], static_cast<uint32_t>(smp[s].t1 + c));
+    }
+  };
   __syncthreads();
-
-  double mu_s[kTpt], nu[kTpt], rmus[kTpt];
-  bool on[kTpt];
-  bool any = false;
-#pragma unroll
-  for (int j = 0; j < kTpt; ++j) {
-    const int x = tile * kBlock * kTpt + j * kBlock + tid;
-    on[j] = x < W;
-    any = any || on[j];
-    mu_s[j] = on[j] ? s_col_mus(J, x % J.nmus) : 0.0;
-    nu[j] = on[j] ? s_slice_nu(J, x / J.nmus, mu, mu_s[j]) : 0.0;
-    rmus[j] = r * mu_s[j];
-  }
-  if (!any) return;
-  Real ar[kTpt][3], am[kTpt][3];
-#pragma unroll
-  for (int j = 0; j < kTpt; ++j)
-    for (int c = 0; c < 3; ++c) ar[j][c] = am[j][c] = Real(0);
+  // With two buffers, the texels of the next sample's rows are loaded while
+  // this one's are used, and a sample takes one barrier.
+  if (kTwo && tid < tw) fetch(0, tid);
   for (int s = 0; s < kMarch; ++s) {
     const SsSample<Real>& S = smp[s];
+    Real* const now = rows + (kTwo ? (s & 1) * 3 * kStaged * tw : 0);
+    if (kStaged > 0) {
+      for (int c = tid; c < tw; c += kB) {
+        if (!kTwo || c != tid) fetch(s, c);
+        const Real w1 = S.wy, w0 = Real(1) - w1;
 #pragma unroll
-    for (int j = 0; j < kTpt; ++j) {
-      if (!on[j]) continue;
-      const double t = fma(S.d, nu[j], rmus[j]);  // r * mu_s + d * nu = r_d * mu_s_d
-      const Real xs = static_cast<Real>((t + S.rho) * S.inv_r);  // mu_s_d - cos(theta_h)
-      // Clamps as max/min, 2 instructions each (the operands are finite; the
-      // ternary form, which also keeps NaNs, compiles to compares and
-      // selects).
-      const Real mus = fmin(fmax(static_cast<Real>(t * S.inv_r), Real(-1)), Real(1));
-      const Real u = fmin(fmax((xs + S.e) * S.inv_span, Real(0)), Real(1));
-      const Real vis = u * u * fma(Real(-2), u, Real(3));
-      Real ts[3];
-      tsun_lookup(J, S, mus, ts);
+        for (int k = 0; k < kStaged; ++k) {
+          const Real* const t = tv[s][k];
+          Real* const v = now + 3 * (k * tw + c);
+          v[0] = fma(w1, Real(b[k].x), w0 * Real(a[k].x)) * t[0];
+          v[1] = fma(w1, Real(b[k].y), w0 * Real(a[k].y)) * t[1];
+          v[2] = fma(w1, Real(b[k].z), w0 * Real(a[k].z)) * t[2];
+        }
+      }
+      if (kTwo && tid < tw && s + 1 < kMarch) fetch(s + 1, tid);
+      __syncthreads();
+    }
+    if (on) {
+      Real u;
+      const Real vis = ss_sun(J, S, fma(s * dx, nu, rmus), &u);
+      const int i0 = min(static_cast<int>(u), tw - 2);
+      const Real w = u - i0;
+      const Real w1 = vis * w, w0 = vis - w1;
+      const Real dr = S.dr, dm = S.dm;
+      // The iterations that are not staged.
+      const uint32_t g0 = static_cast<uint32_t>(S.t0 + i0), g1 = static_cast<uint32_t>(S.t1 + i0);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const Real f = ts[c] * vis;
-        ar[j][c] = fma(f, S.fr[c], ar[j][c]);
-        am[j][c] = fma(f, S.fm[c], am[j][c]);
+      for (int k = kStaged; k < kNit; ++k) {
+        const float4 p = gload32(T[k], g0), q = gload32(T[k], g0 + 1);
+        const float4 pp = gload32(T[k], g1), qq = gload32(T[k], g1 + 1);
+        const Real wy = S.wy, y1 = w1 * wy, x1 = w1 - y1, y0 = w0 * wy, x0 = w0 - y0;
+        const Real* const t = tv[s][k];
+        const Real f[3] = {
+            fma(y1, Real(qq.x), fma(y0, Real(pp.x), fma(x1, Real(q.x), x0 * Real(p.x)))),
+            fma(y1, Real(qq.y), fma(y0, Real(pp.y), fma(x1, Real(q.y), x0 * Real(p.y)))),
+            fma(y1, Real(qq.z), fma(y0, Real(pp.z), fma(x1, Real(q.z), x0 * Real(p.z))))};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const Real h = f[i] * t[i];
+          ar[k][i] = fma(h, dr, ar[k][i]);
+          am[k][i] = fma(h, dm, am[k][i]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kStaged; ++k) {
+        const Real* const v = now + 3 * (k * tw + i0);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const Real f = fma(w1, v[3 + i], w0 * v[i]);
+          ar[k][i] = fma(f, dr, ar[k][i]);
+          am[k][i] = fma(f, dm, am[k][i]);
+        }
       }
     }
+    if (kStaged > 0 && !kTwo) __syncthreads();
   }
+  if (!on) return;
 #pragma unroll
-  for (int j = 0; j < kTpt; ++j) {
-    if (!on[j]) continue;
-    const int x = tile * kBlock * kTpt + j * kBlock + tid;
-    ss_store<kF64>(J, static_cast<int64_t>(row) * W + x, dx, ar[j], am[j]);
-  }
+  for (int k = 0; k < kNit; ++k)
+    ss_store<kF64>((&J)[k], static_cast<int64_t>(row) * W + x, dx, ar[k], am[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1502,9 +1529,9 @@ int blocks_direct_irradiance(const Job& j) {
   return (j.ew * j.eh + kBlock - 1) / kBlock;
 }
 int blocks_single_scattering(const Job& j) {
-  const int w = j.nnu * j.nmus;
-  const int per_block = kBlock * ss_texels_per_thread(w);
-  return ((w + per_block - 1) / per_block) * j.nmu * j.nr;
+  const SsTiling t(j);
+  if (t.nit == 0) return 0;  // served with its group's first
+  return (j.nnu * j.nmus + t.block - 1) / t.block * j.nmu * j.nr;
 }
 int blocks_scattering_density(const Job& j) {
   const SdTile t = kSdTile[j.sd_tile];
@@ -1554,23 +1581,27 @@ hipError_t launch_direct_irradiance(const PassLaunch& p, hipStream_t s) {
                      p.jobs, p.first_block, p.njobs);
   return hipGetLastError();
 }
-template <int kTpt>
-void launch_ss_tpt(const PassLaunch& p, hipStream_t s) {
-  if (kTpt < ss_texels_per_thread(p.min_w) || kTpt > ss_texels_per_thread(p.max_w)) return;
-  const dim3 g(p.total_blocks), b(kBlock);
-  if (p.kinds & kJobsF32)
-    hipLaunchKernelGGL((k_single_scattering<false, kTpt>), g, b, 0, s, p.jobs, p.first_block,
-                       p.njobs);
-  if (p.kinds & kJobsAcc64)
-    hipLaunchKernelGGL((k_single_scattering<true, kTpt>), g, b, 0, s, p.jobs, p.first_block,
-                       p.njobs);
+template <bool kF64, int kNit, int kB>
+void launch_ss(const PassLaunch& p, hipStream_t s) {
+  if (p.ss_kinds & ss_kind(kF64, kNit, kB))
+    hipLaunchKernelGGL((k_single_scattering<kF64, kNit, kB>), dim3(p.total_blocks), dim3(kB),
+                       p.ss_lds, s, p.jobs, p.first_block, p.njobs);
+}
+template <int kB>
+void launch_ss_block(const PassLaunch& p, hipStream_t s) {
+  static_assert(kSsIters == 5, "one launch per group size");
+  launch_ss<false, 1, kB>(p, s);
+  launch_ss<true, 1, kB>(p, s);
+  launch_ss<true, 2, kB>(p, s);
+  launch_ss<true, 3, kB>(p, s);
+  launch_ss<true, 4, kB>(p, s);
+  launch_ss<true, 5, kB>(p, s);
 }
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s) {
-  // One instance per kind of job the launch may hold (accumulator precision,
-  // texels per thread from the packed row widths); each skips the others.
-  launch_ss_tpt<1>(p, s);
-  launch_ss_tpt<2>(p, s);
-  launch_ss_tpt<4>(p, s);
+  // One instance per kind of job (SsTiling); each skips the others.
+  launch_ss_block<64>(p, s);
+  launch_ss_block<kBlock>(p, s);
+  launch_ss_block<2 * kBlock>(p, s);
   return hipGetLastError();
 }
 template <int kChunk, int kB>

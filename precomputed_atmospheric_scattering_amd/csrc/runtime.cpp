@@ -544,9 +544,14 @@ atmo::PassLaunch model_launch(const atmo_model* m, int first_job, int njobs, Pas
   l.dj_kinds = m->spec.half_precision ? atmo::kDjRgb21 : atmo::kDjF32;
   const atmo::Job& j = m->jobs[first_job];
   l.sd_kinds = 1 << atmo::sd_split(j);
-  l.arc_kinds = 0;
-  for (int i = 0; i < njobs; i += atmo::kArcIters)
-    l.arc_kinds |= atmo::arc_kind(m->jobs[first_job + i]);
+  l.ss_kinds = l.arc_kinds = 0;
+  l.ss_lds = 0;
+  for (int i = 0; i < njobs; ++i) {
+    const atmo::Job& ji = m->jobs[first_job + i];
+    if (ji.it % atmo::kArcIters == 0) l.arc_kinds |= atmo::arc_kind(ji);
+    l.ss_kinds |= atmo::ss_kind(ji);
+    l.ss_lds = std::max(l.ss_lds, atmo::ss_lds(ji));
+  }
   l.arc_lds = atmo::arc_lds(j);
   l.tile = p == kSD ? j.sd_tile : (p == kMS ? j.ms_tile : 0);
   return l;
@@ -1458,8 +1463,8 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     l.max_lds_w = 0;
     l.kinds = 0;
     l.dj_kinds = 0;
-    l.sd_kinds = l.arc_kinds = 0;
-    l.arc_lds = 0;
+    l.ss_kinds = l.sd_kinds = l.arc_kinds = 0;
+    l.ss_lds = l.arc_lds = 0;
     int total = 0;
     for (const auto& mj : sel) {
       const atmo::Job& j = models[mj.first]->jobs[mj.second];
@@ -1474,6 +1479,8 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
         l.max_lds_w = std::max(l.max_lds_w, j.nnu * j.nmus);
       l.kinds |= j.acc64 ? atmo::kJobsAcc64 : atmo::kJobsF32;
       l.dj_kinds |= j.half_luts ? atmo::kDjRgb21 : atmo::kDjF32;
+      l.ss_kinds |= atmo::ss_kind(j);
+      l.ss_lds = std::max(l.ss_lds, atmo::ss_lds(j));
       l.sd_kinds |= 1 << atmo::sd_split(j);
       if (j.it % atmo::kArcIters == 0) l.arc_kinds |= atmo::arc_kind(j);
       l.arc_lds = std::max(l.arc_lds, atmo::arc_lds(j));
@@ -1573,6 +1580,8 @@ atmo_status launch_level(const Level& l, const atmo::Job* d_jobs, const int* d_f
   pl.max_lds_w = l.max_lds_w;
   pl.kinds = l.kinds;
   pl.dj_kinds = l.dj_kinds;
+  pl.ss_kinds = l.ss_kinds;
+  pl.ss_lds = l.ss_lds;
   pl.sd_kinds = l.sd_kinds;
   pl.arc_kinds = l.arc_kinds;
   pl.arc_lds = l.arc_lds;

@@ -48,8 +48,8 @@ struct Level {
   Pass pass;
   int order;
   int job_offset, njobs, fb_offset, total_blocks, max_nnu, max_ew, max_w, min_w, max_lds_w,
-      kinds, dj_kinds, sd_kinds, arc_kinds;
-  size_t arc_lds;
+      kinds, dj_kinds, ss_kinds, sd_kinds, arc_kinds;
+  size_t ss_lds, arc_lds;
   int tile;   // SD and MS: the tile shape shared by the level's jobs
 };
 
