@@ -150,7 +150,7 @@ struct Job {
   int half_luts;
   uint2* S16;
   uint2* SM16;
-  // The lookup copy of S and SM (s_quad_taps): 128-byte blocks of quads of
+  // The lookup copy of S and SM (QuadTaps): 128-byte blocks of quads of
   // 4 (S, SM) texel pairs, 8 float4 (FP32) or 4 uint4 (FP16) per quad; null
   // if absent.
   void* Q;
@@ -565,78 +565,41 @@ ATMO_HD QuadAxis quad_axis(double x, int n) {
   }
   return q;
 }
-// The 4 quads of a lookup: f(quad slot, weights of its 4 texels), the
-// weights the products of s_taps in the same order. The slot of a quad is
-// its index in units of quads: the block for FP32 models, 2 x block + (mu
-// tap) for FP16 ones.
-template <class Real, class F>
-ATMO_HD void s_quad_taps(const Job& j, const SCoords& c, F&& f) {
-  const QuadAxis qs = quad_axis(c.nu, j.nnu), qx = quad_axis(c.x_in, j.nmus);
-  double xz = c.z, xy = c.y;
-  Taps tz = axis_taps(xz, j.nr), ty = axis_taps(xy, j.nmu);
-  auto frac = [](double x, int n) {
-    if (!(x >= -1.0)) x = -1.0;
-    if (x > static_cast<double>(n)) x = static_cast<double>(n);
-    return x - floor(x);
-  };
-  const double fz = frac(xz, j.nr), fy = frac(xy, j.nmu);
-  const int zs[2] = {tz.i0, tz.i1};
-  const int ys[2] = {ty.i0, ty.i1};
-  // The mu anchor of the FP16 blocks: its rows clamp(ya) and clamp(ya + 1)
-  // are ty.i0 and ty.i1.
-  const int ya = quad_axis(xy, j.nmu).a;
-  const bool half = j.half_luts != 0;
-  const Real wz[2] = {static_cast<Real>(1.0 - fz), static_cast<Real>(fz)};
-  const Real wy[2] = {static_cast<Real>(1.0 - fy), static_cast<Real>(fy)};
-  const Real wx[2] = {static_cast<Real>(1.0 - qx.w), static_cast<Real>(qx.w)};
-  const Real wsl[2] = {static_cast<Real>(1.0 - qs.w), static_cast<Real>(qs.w)};
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) {
-      Real w[4];
-      for (int e = 0; e < 2; ++e)
-        for (int q = 0; q < 2; ++q) w[2 * e + q] = wz[a] * wy[b] * wx[e] * wsl[q];
-      const int64_t slot =
-          half ? 2 * lookup_copy_block(j, zs[a], ya + 1, qs.a, qx.a) + b
-               : lookup_copy_block(j, zs[a], ys[b], qs.a, qx.a);
-      f(slot, w);
-    }
-}
-struct F32Quads {
-  const float4* q;  // 8 float4 per quad: (S, SM) of its 4 texels
-  ATMO_HD void load(int64_t quad, int k, float4* s, float4* m) const {
-    *s = gload(q, 8 * quad + 2 * k);
-    *m = gload(q, 8 * quad + 2 * k + 1);
+// The quads of a lookup, in the order of s_taps: quad 2 a + b of the taps
+// zs[a], ys[b], its texel 2 e + q with weight wz[a] wy[b] wx[e] ws[q]. FP32
+// models: line[2 a + b] is the quad's block; FP16 ones: line[a] is the block
+// of quads 2 a and 2 a + 1.
+template <class Real>
+struct QuadTaps {
+  uint32_t line[4];
+  Real wz[2], wy[2], wx[2], ws[2];
+  ATMO_HD QuadTaps(const Job& j, const SCoords& c) {
+    const QuadAxis qs = quad_axis(c.nu, j.nnu), qx = quad_axis(c.x_in, j.nmus);
+    const Taps tz = axis_taps(c.z, j.nr), ty = axis_taps(c.y, j.nmu);
+    auto frac = [](double x, int n) {
+      if (!(x >= -1.0)) x = -1.0;
+      if (x > static_cast<double>(n)) x = static_cast<double>(n);
+      return x - floor(x);
+    };
+    const double fz = frac(c.z, j.nr), fy = frac(c.y, j.nmu);
+    const int zs[2] = {tz.i0, tz.i1}, ys[2] = {ty.i0, ty.i1};
+    // The mu anchor of the FP16 blocks: its rows clamp(ya) and clamp(ya + 1)
+    // are ty.i0 and ty.i1.
+    const int ya = quad_axis(c.y, j.nmu).a;
+    for (int a = 0; a < 2; ++a)
+      for (int b = 0; b < 2; ++b)
+        line[j.half_luts ? a : 2 * a + b] = static_cast<uint32_t>(
+            lookup_copy_block(j, zs[a], j.half_luts ? ya + 1 : ys[b], qs.a, qx.a));
+    wz[0] = static_cast<Real>(1.0 - fz);
+    wz[1] = static_cast<Real>(fz);
+    wy[0] = static_cast<Real>(1.0 - fy);
+    wy[1] = static_cast<Real>(fy);
+    wx[0] = static_cast<Real>(1.0 - qx.w);
+    wx[1] = static_cast<Real>(qx.w);
+    ws[0] = static_cast<Real>(1.0 - qs.w);
+    ws[1] = static_cast<Real>(qs.w);
   }
-  ATMO_HD float4 scale_s() const { return make_float4(1.0f, 1.0f, 1.0f, 1.0f); }
-  ATMO_HD float4 scale_m() const { return make_float4(1.0f, 1.0f, 1.0f, 1.0f); }
 };
-// FP16 quads: stored values, scaled after the sums as for F16Texels.
-struct F16Quads {
-  const uint4* q;  // 4 uint4 per quad: S and SM of a texel as 4 x FP16 each
-  float4 inv_s, inv_m;
-  ATMO_HD void load(int64_t quad, int k, float4* s, float4* m) const {
-    const uint4 u = gload(q, 4 * quad + k);
-    *s = unpack_half4(make_uint2(u.x, u.y));
-    *m = unpack_half4(make_uint2(u.z, u.w));
-  }
-  ATMO_HD float4 scale_s() const { return inv_s; }
-  ATMO_HD float4 scale_m() const { return inv_m; }
-};
-template <class Quads>
-ATMO_HD void s_lookup_quads_d(const Job& j, const Quads& lut, const SCoords& c, D4* s,
-                              D4* m) {
-  D4 as{0.0, 0.0, 0.0, 0.0}, am{0.0, 0.0, 0.0, 0.0};
-  s_quad_taps<double>(j, c, [&](int64_t quad, const double* w) {
-    for (int k = 0; k < 4; ++k) {
-      float4 vs, vm;
-      lut.load(quad, k, &vs, &vm);
-      acc_d4(&as, w[k], vs);
-      acc_d4(&am, w[k], vm);
-    }
-  });
-  *s = scaled(as, lut.scale_s());
-  *m = scaled(am, lut.scale_m());
-}
 
 // The same lookups with FP32 weights and sums, for lookups whose result is
 // not a difference of two lookups (GetSkyRadiance): relative error about
@@ -654,22 +617,6 @@ ATMO_HD D4 s_lookup_f(const Job& j, const Texels& lut, const SCoords& c) {
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   s_taps<float>(j, c, [&](int64_t i, float wt) { acc_f4(&acc, wt, lut[i]); });
   return to_d4(scaled(acc, lut.scale()));
-}
-
-template <class Quads>
-ATMO_HD void s_lookup_quads_f(const Job& j, const Quads& lut, const SCoords& c, D4* s,
-                              D4* m) {
-  float4 as = make_float4(0.0f, 0.0f, 0.0f, 0.0f), am = as;
-  s_quad_taps<float>(j, c, [&](int64_t quad, const float* w) {
-    for (int k = 0; k < 4; ++k) {
-      float4 vs, vm;
-      lut.load(quad, k, &vs, &vm);
-      acc_f4(&as, w[k], vs);
-      acc_f4(&am, w[k], vm);
-    }
-  });
-  *s = to_d4(scaled(as, lut.scale_s()));
-  *m = to_d4(scaled(am, lut.scale_m()));
 }
 
 // Real: the type of the weights and sums (double: exact FP64 weights;
@@ -707,21 +654,20 @@ ATMO_HD D4 t_lookup_d(const Job& j, const float4* T, double r, double mu) {
   return t_lookup_r<double>(j, T, r, mu);
 }
 
-// functions.glsl:493-519 in FP64 arithmetic.
-ATMO_HD D4 transmittance_d(const Job& j, const float4* T, double r, double mu,
-                           double d, bool ground) {
+// functions.glsl:493-519 in FP64 arithmetic; 'here' is the lookup at
+// (r, mu), or at (r, -mu) for ground rays.
+ATMO_HD D4 transmittance_from_d(const Job& j, const float4* T, D4 here, double r, double mu,
+                                double d, bool ground) {
   const double r_d = clamp_radius(j, sqrt(d * d + 2.0 * r * mu * d + r * r));
   const double mu_d = clamp_cos((r * mu + d) / r_d);
-  D4 num, den;
-  if (ground) {
-    num = t_lookup_d(j, T, r_d, -mu_d);
-    den = t_lookup_d(j, T, r, -mu);
-  } else {
-    num = t_lookup_d(j, T, r, mu);
-    den = t_lookup_d(j, T, r_d, mu_d);
-  }
+  const D4 there = t_lookup_d(j, T, r_d, ground ? -mu_d : mu_d);
+  const D4 num = ground ? there : here, den = ground ? here : there;
   auto m1 = [](double v) { return v < 1.0 ? v : 1.0; };
   return D4{m1(num.x / den.x), m1(num.y / den.y), m1(num.z / den.z), 0.0};
+}
+ATMO_HD D4 transmittance_d(const Job& j, const float4* T, double r, double mu,
+                           double d, bool ground) {
+  return transmittance_from_d(j, T, t_lookup_d(j, T, r, ground ? -mu : mu), r, mu, d, ground);
 }
 
 // functions.glsl:552-563 in FP64 arithmetic (Real: the lookup's weights and

@@ -7,6 +7,8 @@
 // of two nearby lookups in GetSkyRadianceToPoint keeps the texels' precision.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "atmo_device.h"
 #include "kernels.h"
 
@@ -47,34 +49,119 @@ __device__ __forceinline__ D4 extrapolated_mie(const Job& J, D4 s) {
             s.z * k * (J.mie_sca[2] / J.rayleigh[2]), 0.0};
 }
 
+__device__ __forceinline__ void acc_q(D4* acc, double w, float4 v) { acc_d4(acc, w, v); }
+__device__ __forceinline__ void acc_q(float4* acc, float w, float4 v) { acc_f4(acc, w, v); }
+__device__ __forceinline__ D4 as_d4(D4 v) { return v; }
+__device__ __forceinline__ D4 as_d4(float4 v) { return to_d4(v); }
+
+// 16-byte parts of lookup copy lines that a wave holds in LDS: one line of
+// each lane.
+constexpr int kLineParts = 8;
+constexpr int kStageParts = 64 * kLineParts;
+// Lanes whose first line is their neighbour's from which on lanes load their
+// own lines (neighbouring pixels of a frame).
+constexpr int kNearLanes = 32;
+
+__device__ __forceinline__ float4 as_floats(uint4 a) {
+  return make_float4(__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z),
+                     __uint_as_float(a.w));
+}
+
+// The lookup of S and SM in the lookup copy for the rays of a wave, whose
+// lanes are all active. A ray reads 2 (FP16) or 4 lines of 128 bytes at random.
+// Read by its own lane, a line takes 8 loads, each of them 64 lines for the
+// wave: a scattered 16-byte load cost 50 cycles of the address unit, which
+// was busy 70% of the time with the vector units at 49% and 2 waves per SIMD
+// (226 VGPRs hold the loads in flight). Here 8 lanes read a line together, so
+// that a load takes 8 whole lines, and each lane gets its own from LDS. Part k
+// of a line is at k ^ (lane % 8), so that neighbouring lanes read different
+// banks. Where most lanes' lines are their neighbours' (the pixels of a frame),
+// the lanes load their own.
+// 2.07M rays on MI355X, own lines | shared, us: GetSkyRadiance scattered 134 |
+// 97 FP32, 85 | 78 FP16; GetSkyRadianceToPoint scattered 307 | 198 and 212 |
+// 176, pixels 177 | 152 and 150 | 152.
+template <class Real, bool kHalf>
+__device__ __forceinline__ void lookup_lines(const Job& J, const SCoords& c, uint4* stage,
+                                             D4* s, D4* m) {
+  using Acc = typename std::conditional<sizeof(Real) == 8, D4, float4>::type;
+  const QuadTaps<Real> t(J, c);
+  const uint4* __restrict__ lines = static_cast<const uint4*>(J.Q);
+  const int lane = threadIdx.x & 63, group = lane / kLineParts, part = lane % kLineParts;
+  constexpr int kLines = kHalf ? 2 : 4;
+  Acc as{}, am{};
+  // Part k of line n of the lane.
+  auto add = [&](int n, int k, uint4 u) {
+    const int a = kHalf ? n : n / 2, b = kHalf ? k / 4 : n % 2, texel = kHalf ? k % 4 : k / 2;
+    const Real w = t.wz[a] * t.wy[b] * t.wx[texel / 2] * t.ws[texel % 2];
+    if (kHalf) {
+      acc_q(&as, w, unpack_half4(make_uint2(u.x, u.y)));
+      acc_q(&am, w, unpack_half4(make_uint2(u.z, u.w)));
+    } else {
+      acc_q(k % 2 ? &am : &as, w, as_floats(u));
+    }
+  };
+  if (__popcll(__ballot(t.line[0] == __shfl_xor(t.line[0], 1))) >= kNearLanes) {
+#pragma unroll
+    for (int n = 0; n < kLines; ++n)
+#pragma unroll
+      for (int k = 0; k < kLineParts; ++k)
+        add(n, k, gload(lines, static_cast<int64_t>(t.line[n]) * kLineParts + k));
+  } else {
+    uint4 v[kLineParts];
+    auto fetch = [&](int n) {
+#pragma unroll
+      for (int k = 0; k < kLineParts; ++k) {
+        const uint32_t line = __shfl(t.line[n], kLineParts * k + group);
+        v[k] = gload(lines, static_cast<int64_t>(line) * kLineParts + part);
+      }
+    };
+    fetch(0);
+#pragma unroll
+    for (int n = 0; n < kLines; ++n) {
+#pragma unroll
+      for (int k = 0; k < kLineParts; ++k)
+        stage[(kLineParts * k + group) * kLineParts + (part ^ group)] = v[k];
+      // (The lanes of a wave run in step and its LDS accesses in order.)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (n + 1 < kLines) fetch(n + 1);
+#pragma unroll
+      for (int k = 0; k < kLineParts; ++k)
+        add(n, k, stage[lane * kLineParts + (k ^ part)]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  if (kHalf) {
+    // Stored values, scaled after the sums as for F16Texels.
+    const float* sc = J.scales;
+    as = scaled(as, make_float4(1.0f / sc[0], 1.0f / sc[1], 1.0f / sc[2], 1.0f / sc[3]));
+    am = scaled(am, make_float4(1.0f / sc[4], 1.0f / sc[5], 1.0f / sc[6], 0.0f));
+  }
+  *s = as_d4(as);
+  *m = as_d4(am);
+}
+
 // functions.glsl:1658-1690. kF32: FP32 tap weights and sums (lookups whose
-// result is not a difference of two lookups); otherwise FP64.
-template <bool kF32>
+// result is not a difference of two lookups); otherwise FP64. kLines: S and SM
+// are separate; then all lanes of the wave call it, with the wave's kStageParts
+// parts of LDS.
+template <bool kF32, bool kLines>
 __device__ D4 combined_scattering(const Job& J, double r, double mu, double mu_s,
-                                  double nu, bool ground, D4* single_mie) {
+                                  double nu, bool ground, uint4* stage, D4* single_mie) {
+  using Real = typename std::conditional<kF32, float, double>::type;
   const SCoords c = s_coords(J, r, mu, mu_s, nu, ground);
   auto lookup = [&](const auto& lut) {
     return kF32 ? s_lookup_f(J, lut, c) : s_lookup_d(J, lut, c);
   };
-  auto lookup_quads = [&](const auto& lut, D4* s, D4* m) {
-    if (kF32)
-      s_lookup_quads_f(J, lut, c, s, m);
-    else
-      s_lookup_quads_d(J, lut, c, s, m);
-  };
   D4 s;
-  if (J.Q != nullptr && !J.combined) {
+  if (kLines && J.Q != nullptr) {
     // Lookup copy: the S and SM texels of the 4 (nu, mu_s) taps of each
     // (r, mu) tap in one contiguous quad.
-    if (J.half_luts) {
-      const float* sc = J.scales;
-      const F16Quads qt{static_cast<const uint4*>(J.Q),
-                        make_float4(1.0f / sc[0], 1.0f / sc[1], 1.0f / sc[2], 1.0f / sc[3]),
-                        make_float4(1.0f / sc[4], 1.0f / sc[5], 1.0f / sc[6], 0.0f)};
-      lookup_quads(qt, &s, single_mie);
-    } else {
-      lookup_quads(F32Quads{static_cast<const float4*>(J.Q)}, &s, single_mie);
-    }
+    if (J.half_luts)
+      lookup_lines<Real, true>(J, c, stage, &s, single_mie);
+    else
+      lookup_lines<Real, false>(J, c, stage, &s, single_mie);
     *single_mie = rgb(*single_mie);
     return s;
   }
@@ -83,16 +170,16 @@ __device__ D4 combined_scattering(const Job& J, double r, double mu, double mu_s
     const F16Texels st{J.S16, make_float4(1.0f / sc[0], 1.0f / sc[1], 1.0f / sc[2],
                                           1.0f / sc[3])};
     s = lookup(st);
-    if (!J.combined) {
+    if (kLines) {
       const F16Texels mt{J.SM16, make_float4(1.0f / sc[4], 1.0f / sc[5], 1.0f / sc[6],
                                              0.0f)};
       *single_mie = rgb(lookup(mt));
     }
   } else {
     s = lookup(F32Texels{J.S});
-    if (!J.combined) *single_mie = rgb(lookup(F32Texels{J.SM}));
+    if (kLines) *single_mie = rgb(lookup(F32Texels{J.SM}));
   }
-  if (J.combined) *single_mie = extrapolated_mie(J, s);
+  if (!kLines) *single_mie = extrapolated_mie(J, s);
   return s;
 }
 
@@ -108,13 +195,24 @@ __device__ __forceinline__ D4 shade(const Job& J, D4 scat, D4 mie, double nu,
   return l;
 }
 
-__global__ __launch_bounds__(kBlock) void k_sky_radiance(
+// kLines: for models with separate S and SM (combined_scattering). Three waves
+// per SIMD take 168 VGPRs with lines (175 unbounded, 8% slower); without, the
+// loads in flight of fewer waves are worth more (FP16, scattered: 121 us for
+// 2.07M rays with 2, 131 with 3).
+template <bool kLines>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kLines ? 3 : 2))) void
+k_sky_radiance(
     const Job* __restrict__ job, int64_t n, const float* __restrict__ camera,
     const float* __restrict__ view_ray, const float* __restrict__ shadow_length,
     const float* __restrict__ sun_direction, float* __restrict__ radiance,
     float* __restrict__ transmittance_out, int luminance) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
+  __shared__ uint4 stage_of[kLines ? kBlock / 64 : 1][kLines ? kStageParts : 1];
+  uint4* const stage = stage_of[kLines ? threadIdx.x / 64 : 0];
+  // All lanes of a wave take part in the lookups of lines: those past the end
+  // repeat the last ray and store nothing.
+  const int64_t ray = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (!kLines && ray >= n) return;
+  const int64_t i = ray < n ? ray : n - 1;
   const Job& J = *job;
   D3 cam = load3(camera, i);
   const D3 v = load3(view_ray, i);
@@ -124,45 +222,63 @@ __global__ __launch_bounds__(kBlock) void k_sky_radiance(
   double r = sqrt(dot3(cam, cam));
   double rmu = dot3(cam, v);
   const double to_top = -rmu - sqrt(rmu * rmu - r * r + J.rt * J.rt);
+  bool space = false;
   if (to_top > 0.0) {
     cam = D3{cam.x + v.x * to_top, cam.y + v.y * to_top, cam.z + v.z * to_top};
     r = J.rt;
     rmu += to_top;
   } else if (r > J.rt) {
-    store3(transmittance_out, i, D4{1.0, 1.0, 1.0, 0.0});
-    store3(radiance, i, D4{0.0, 0.0, 0.0, 0.0});
-    return;
+    // In space, looking past the atmosphere.
+    if (!kLines) {
+      store3(transmittance_out, i, D4{1.0, 1.0, 1.0, 0.0});
+      store3(radiance, i, D4{0.0, 0.0, 0.0, 0.0});
+      return;
+    }
+    space = true;
+    r = J.rt;
+    rmu = r;
   }
   const double mu = rmu / r;
   const double mu_s = dot3(cam, sd) / r;
   const double nu = dot3(v, sd);
   const bool ground = hits_ground(J, r, mu);
-  const D4 t = ground ? D4{0.0, 0.0, 0.0, 0.0} : t_lookup_d(J, J.T, r, mu);
-  D4 mie, scat;
-  if (shadow == 0.0) {
-    scat = rgb(combined_scattering<true>(J, r, mu, mu_s, nu, ground, &mie));
-  } else {
+  const D4 zero{0.0, 0.0, 0.0, 0.0};
+  const D4 t = ground ? zero : t_lookup_d(J, J.T, r, mu);
+  double r_p = r, mu_p = mu, mu_s_p = mu_s;
+  if (shadow != 0.0) {
     // Light shafts (functions.glsl:1746-1766).
     const double d = shadow;
-    const double r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
-    const double mu_p = (r * mu + d) / r_p;
-    const double mu_s_p = (r * mu_s + d * nu) / r_p;
-    scat = rgb(combined_scattering<true>(J, r_p, mu_p, mu_s_p, nu, ground, &mie));
+    r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
+    mu_p = (r * mu + d) / r_p;
+    mu_s_p = (r * mu_s + d * nu) / r_p;
+  }
+  D4 mie;
+  D4 scat = rgb(combined_scattering<true, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage,
+                                                  &mie));
+  if (ray >= n) return;
+  if (shadow != 0.0) {
     const D4 st = transmittance_d(J, J.T, r, mu, shadow, ground);
     scat = mul(scat, st);
     mie = mul(mie, st);
   }
-  store3(radiance, i, shade(J, scat, mie, nu, luminance));
-  store3(transmittance_out, i, t);
+  store3(radiance, i, space ? zero : shade(J, scat, mie, nu, luminance));
+  store3(transmittance_out, i, space ? D4{1.0, 1.0, 1.0, 0.0} : t);
 }
 
-__global__ __launch_bounds__(kBlock) void k_sky_radiance_to_point(
+// (Two waves per SIMD: with lines its FP64 sums take 227 VGPRs, and 3 spill;
+// without, 3 waves make scattered lookups 4% slower.)
+template <bool kLines>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_sky_radiance_to_point(
     const Job* __restrict__ job, int64_t n, const float* __restrict__ camera,
     const float* __restrict__ point, const float* __restrict__ shadow_length,
     const float* __restrict__ sun_direction, float* __restrict__ radiance,
     float* __restrict__ transmittance_out, int luminance) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
+  __shared__ uint4 stage_of[kLines ? kBlock / 64 : 1][kLines ? kStageParts : 1];
+  uint4* const stage = stage_of[kLines ? threadIdx.x / 64 : 0];
+  const int64_t ray = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (!kLines && ray >= n) return;
+  const int64_t i = ray < n ? ray : n - 1;  // as in k_sky_radiance
   const Job& J = *job;
   D3 cam = load3(camera, i);
   const D3 p = load3(point, i);
@@ -186,21 +302,25 @@ __global__ __launch_bounds__(kBlock) void k_sky_radiance_to_point(
   const D3 pc = D3{p.x - cam.x, p.y - cam.y, p.z - cam.z};
   double d = sqrt(dot3(pc, pc));
   const bool ground = hits_ground(J, r, mu);
-  const D4 t = transmittance_d(J, J.T, r, mu, d, ground);
+  // Both transmittances below are quotients with the lookup at the camera.
+  const D4 here = t_lookup_d(J, J.T, r, ground ? -mu : mu);
+  const D4 t = transmittance_from_d(J, J.T, here, r, mu, d, ground);
   D4 mie;
-  D4 scat = rgb(combined_scattering<false>(J, r, mu, mu_s, nu, ground, &mie));
+  D4 scat = rgb(combined_scattering<false, kLines>(J, r, mu, mu_s, nu, ground, stage, &mie));
   // functions.glsl:1831-1840
   d = d - shadow > 0.0 ? d - shadow : 0.0;
   const double r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
   const double mu_p = (r * mu + d) / r_p;
   const double mu_s_p = (r * mu_s + d * nu) / r_p;
   D4 mie_p;
-  const D4 scat_p = rgb(combined_scattering<false>(J, r_p, mu_p, mu_s_p, nu, ground, &mie_p));
+  const D4 scat_p =
+      rgb(combined_scattering<false, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage, &mie_p));
+  if (ray >= n) return;
   D4 st = t;
-  if (shadow > 0.0) st = transmittance_d(J, J.T, r, mu, d, ground);
+  if (shadow > 0.0) st = transmittance_from_d(J, J.T, here, r, mu, d, ground);
   scat = sub(scat, mul(st, scat_p));
   mie = sub(mie, mul(st, mie_p));
-  if (J.combined) mie = extrapolated_mie(J, D4{scat.x, scat.y, scat.z, mie.x});
+  if (!kLines) mie = extrapolated_mie(J, D4{scat.x, scat.y, scat.z, mie.x});
   // functions.glsl:1857-1859
   mie = scale(mie, smoothstep_d(0.0, 0.01, mu_s));
   store3(radiance, i, shade(J, scat, mie, nu, luminance));
@@ -291,19 +411,19 @@ inline unsigned grid_for(int64_t n) {
 
 }  // namespace
 
-hipError_t launch_sky_radiance(const Job* job, int64_t n, const float* camera,
+hipError_t launch_sky_radiance(const Job* job, bool combined, int64_t n, const float* camera,
                                const float* view_ray,
                                const float* shadow_length,
                                const float* sun_direction, float* radiance,
                                float* transmittance, int luminance, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sky_radiance, dim3(grid_for(n)), dim3(kBlock), 0, s, job, n,
-                     camera, view_ray, shadow_length, sun_direction, radiance,
-                     transmittance, luminance);
+  const auto kernel = combined ? k_sky_radiance<false> : k_sky_radiance<true>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, job, n, camera, view_ray,
+                     shadow_length, sun_direction, radiance, transmittance, luminance);
   return hipGetLastError();
 }
 
-hipError_t launch_sky_radiance_to_point(const Job* job, int64_t n,
+hipError_t launch_sky_radiance_to_point(const Job* job, bool combined, int64_t n,
                                         const float* camera,
                                         const float* point,
                                         const float* shadow_length,
@@ -311,9 +431,9 @@ hipError_t launch_sky_radiance_to_point(const Job* job, int64_t n,
                                         float* radiance, float* transmittance,
                                         int luminance, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sky_radiance_to_point, dim3(grid_for(n)), dim3(kBlock), 0, s,
-                     job, n, camera, point, shadow_length, sun_direction, radiance,
-                     transmittance, luminance);
+  const auto kernel = combined ? k_sky_radiance_to_point<false> : k_sky_radiance_to_point<true>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, job, n, camera, point,
+                     shadow_length, sun_direction, radiance, transmittance, luminance);
   return hipGetLastError();
 }
 

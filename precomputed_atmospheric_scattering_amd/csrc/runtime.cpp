@@ -1155,9 +1155,9 @@ static atmo_status sky(const atmo_model* m, int64_t n, const float* camera,
   if (n > 0 && (!camera || !view_ray || !shadow_length || !sun_direction || !radiance ||
                 !transmittance))
     return fail(ATMO_ERROR_INVALID_ARGUMENT, "NULL array");
-  return check_launch(atmo::launch_sky_radiance(query_job(m), n, camera, view_ray,
-                                                shadow_length, sun_direction, radiance,
-                                                transmittance, luminance,
+  return check_launch(atmo::launch_sky_radiance(query_job(m), m->spec.combined, n, camera,
+                                                view_ray, shadow_length, sun_direction,
+                                                radiance, transmittance, luminance,
                                                 static_cast<hipStream_t>(stream)),
                       "sky radiance");
 }
@@ -1171,8 +1171,8 @@ static atmo_status sky_to_point(const atmo_model* m, int64_t n, const float* cam
                 !transmittance))
     return fail(ATMO_ERROR_INVALID_ARGUMENT, "NULL array");
   return check_launch(atmo::launch_sky_radiance_to_point(
-                          query_job(m), n, camera, point, shadow_length, sun_direction,
-                          radiance, transmittance, luminance,
+                          query_job(m), m->spec.combined, n, camera, point, shadow_length,
+                          sun_direction, radiance, transmittance, luminance,
                           static_cast<hipStream_t>(stream)),
                       "sky radiance to point");
 }
