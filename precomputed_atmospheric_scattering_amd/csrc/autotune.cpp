@@ -219,7 +219,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     pl.arc_lds = 0;
     pl.tile = tile;
     auto launch = [&]() {
-      return pass == kSD ? atmo::launch_scattering_density(pl, s)
+      return pass == kSD ? atmo::launch_scattering_density(pl, 2, s)
                          : atmo::launch_multiple_scattering(pl, s);
     };
     ATMO_TRY(check_launch(launch(), "tuning launch"));  // warm-up

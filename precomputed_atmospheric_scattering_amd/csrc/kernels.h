@@ -64,6 +64,20 @@ ATMO_HD int sd_default_tile(int nmu, int nnu) {
   return nmu * ((nnu + 3) / 4) <= 256 ? 3 : 0;
 }
 
+// FP16-storage models of up to kFixedTexels texels keep the order in which
+// their sums of float32 were always made. FP16 rounding turns a difference of
+// 1e-7 of a sum into one of 1e-3 in some texels (arc sums for the orders >= 3:
+// the last bit of 9e-5 of the texels at 1.05M), and GetSkyRadianceToPoint, a
+// difference of two lookups, into up to 4e-3 of the rms radiance: within the
+// format's error, but a model then shades differently from LUT files and from
+// other models made before. Beyond that size the time decides: at 16.8M texels
+// and 8 orders the arc sums save 57 ms of 212, at 1.05M and 4 orders 1.4 of 6.2.
+constexpr int64_t kFixedTexels = int64_t{1} << 22;
+ATMO_HD bool fixed_sums(const Job& j) {
+  return j.half_luts != 0 &&
+         static_cast<int64_t>(j.nr) * j.nmu * j.nmus * j.nnu <= kFixedTexels;
+}
+
 // Grids too small to fill the GPU at 4 outputs per thread: several threads
 // share an output, each summing some of the zenith angles, whatever the tile
 // shape. A job takes the first of these whose 'texels' it does not exceed (of
@@ -88,7 +102,7 @@ constexpr SdSplit kSdSplit[kSdSplits] = {
 // The job's index into kSdSplit, or kSdSplits.
 ATMO_HD int sd_split(const Job& j) {
   const int64_t n = static_cast<int64_t>(j.nr) * j.nmu * j.nmus * j.nnu * j.niter;
-  int i = 0;
+  int i = fixed_sums(j) ? kSdSplits : 0;
   while (i < kSdSplits && n > kSdSplit[i].texels) ++i;
   return i;
 }
@@ -113,11 +127,13 @@ ATMO_HD size_t ss_row_bytes(const Job& j, int nit, int block) {
 struct SsTiling {
   int block;
   int nit;  // 0: the job is served by the blocks of an earlier iteration
+  bool fixed;  // FP32 job of fixed_sums: k_single_scattering_fixed instead
   ATMO_HD explicit SsTiling(const Job& j) {
     const int w = j.nnu * j.nmus, most = j.niter < kSsIters ? j.niter : kSsIters;
     block = w > kBlock ? 2 * kBlock : (w > 64 ? kBlock : 64);
     const int64_t blocks = static_cast<int64_t>(j.nr) * j.nmu * ((w + block - 1) / block);
     nit = 1;
+    fixed = fixed_sums(j) && !j.acc64;
     // Iterations share a block once that leaves two blocks per CU.
     if (most > 1 && ss_row_bytes(j, most, block) <= kSsRowBytes && blocks >= kSsGroupBlocks) {
       const int left = j.niter - j.it;
@@ -129,9 +145,10 @@ struct SsTiling {
 constexpr int ss_kind(bool f64, int nit, int block) {
   return 1 << ((f64 ? nit : 0) + (block > kBlock ? 2 : (block == kBlock ? 1 : 0)) * (kSsIters + 1));
 }
+constexpr int kSsFixed = 1 << (3 * (kSsIters + 1));
 ATMO_HD int ss_kind(const Job& j) {
   const SsTiling t(j);
-  return t.nit == 0 ? 0 : ss_kind(j.acc64 != 0, t.nit, t.block);
+  return t.nit == 0 ? 0 : t.fixed ? kSsFixed : ss_kind(j.acc64 != 0, t.nit, t.block);
 }
 inline size_t ss_lds(const Job& j) {
   const SsTiling t(j);
@@ -235,10 +252,11 @@ hipError_t launch_optical_depth(const PassLaunch& p, hipStream_t s);
 hipError_t launch_transmittance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_direct_irradiance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s);
-// The scattering density of order 2, and that of an order >= 3. In the
+// The scattering density direction by direction (order 2, and the orders >= 3
+// of the fixed_sums jobs), and that of an order >= 3 by arc sums. In the
 // latter the jobs of a model's Precompute iterations follow each other in
 // p.jobs, and the blocks of the first of every kArcIters serve all of them.
-hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s);
+hipError_t launch_scattering_density(const PassLaunch& p, int order, hipStream_t s);
 hipError_t launch_density_arcs(const PassLaunch& p, hipStream_t s);
 // 'order' is the order of the scattering read by the pass (>= 1).
 hipError_t launch_indirect_irradiance(const PassLaunch& p, int order,

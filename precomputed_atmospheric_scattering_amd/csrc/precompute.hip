@@ -302,7 +302,7 @@ k_single_scattering(
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
   const SsTiling tl(J);
-  if ((J.acc64 != 0) != kF64 || tl.nit != kNit || tl.block != kB) return;
+  if ((J.acc64 != 0) != kF64 || tl.fixed || tl.nit != kNit || tl.block != kB) return;
   const int W = J.nnu * J.nmus;
   const int lb = blockIdx.x - first_block[ji];
   const int tiles = (W + kB - 1) / kB;
@@ -410,6 +410,159 @@ k_single_scattering(
     ss_store<kF64>((&J)[k], static_cast<int64_t>(row) * W + x, dx, ar[k], am[k]);
 }
 
+// The FP32 single scattering of the fixed_sums jobs: each texel gathers its
+// four transmittance texels and interpolates along mu_s first. kTpt: texels
+// per thread, ss_texels_per_thread(W) of the job.
+struct SsFixedSample {
+  double d;         // distance along the view ray
+  double inv_r;     // 1 / r_d
+  double rho;       // sqrt(r_d^2 - rb^2)
+  float r;          // r_d
+  float c;          // rt^2 - r_d^2
+  float dmin;       // rt - r_d
+  float inv_range;  // 1 / (rho + H - dmin)
+  float e;          // sin(theta_h) * sun angular radius
+  float inv_span;   // 1 / (2 e)
+  float wy;
+  int t0, t1;       // first texels of the transmittance LUT rows of r_d
+  float fr[3];      // trapezoid weight * view transmittance * Rayleigh density
+  float fm[3];      // same with the Mie density
+};
+
+// functions.glsl:402-421 at (r_d, mu_s_d): DistanceToTopAtmosphereBoundary
+// in the cancellation-free form, the LUT column coordinate, and the bilinear
+// transmittance lookup (functions.glsl:473-480).
+__device__ __forceinline__ void tsun_lookup(const Job& J, const SsFixedSample& S,
+                                            float mus, float o[3]) {
+  const float tt = S.r * mus;
+  const float sq = sqrt_f(fmaf(tt, tt, S.c));
+  const float dd = tt > 0.0f ? S.c * rcp_f(sq + tt) : sq - tt;
+  const float xm = (dd - S.dmin) * S.inv_range;
+  const float ut = clamp_index_coord(xm * static_cast<float>(J.tw - 1),
+                                     static_cast<float>(J.tw - 1));
+  float w;
+  const int i0 = split_coord(ut, &w);
+  const int i1 = min(i0 + 1, J.tw - 1);
+  const float4* __restrict__ T = J.T;
+  const uint32_t r0 = static_cast<uint32_t>(S.t0), r1 = static_cast<uint32_t>(S.t1);
+  const float4 a = gload32(T, r0 + i0), b = gload32(T, r0 + i1);
+  const float4 c = gload32(T, r1 + i0), d = gload32(T, r1 + i1);
+  const float wy1 = S.wy, wy0 = 1.0f - S.wy;
+  o[0] = fmaf(wy1, fmaf(w, d.x - c.x, c.x), wy0 * fmaf(w, b.x - a.x, a.x));
+  o[1] = fmaf(wy1, fmaf(w, d.y - c.y, c.y), wy0 * fmaf(w, b.y - a.y, a.y));
+  o[2] = fmaf(wy1, fmaf(w, d.z - c.z, c.z), wy0 * fmaf(w, b.z - a.z, a.z));
+}
+
+__host__ __device__ inline int ss_texels_per_thread(int w) {
+  return w >= 4 * kBlock ? 4 : (w >= 2 * kBlock ? 2 : 1);
+}
+
+template <int kTpt>
+__global__ __launch_bounds__(kBlock) void k_single_scattering_fixed(
+    const Job* __restrict__ jobs, const int* __restrict__ first_block,
+    int njobs) {
+  __shared__ SsFixedSample smp[kMarch];
+  const int ji = find_job(first_block, njobs, blockIdx.x);
+  const Job& J = jobs[ji];
+  if (!SsTiling(J).fixed) return;
+  const int W = J.nnu * J.nmus;
+  if (ss_texels_per_thread(W) != kTpt) return;
+  const int lb = blockIdx.x - first_block[ji];
+  const int tiles = (W + kBlock * kTpt - 1) / (kBlock * kTpt);
+  const int tile = lb % tiles;
+  const int row = lb / tiles;  // z * nmu + y
+  const int y = row % J.nmu, z = row / J.nmu;
+  const int tid = threadIdx.x;
+
+  double r, rho, mu;
+  bool ground;
+  s_layer_r(J, z, &r, &rho);
+  s_row_mu(J, y, r, rho, &mu, &ground);
+  const double dx = dist_nearest(J, r, mu, ground) / (kMarch - 1);
+
+  if (tid < kMarch) {
+    SsFixedSample& S = smp[tid];
+    const double d = tid * dx;
+    const double r_d = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
+    double tv[3];
+    const float3 t = transmittance(J, J.T, r, mu, d, ground);
+    tv[0] = t.x;
+    tv[1] = t.y;
+    tv[2] = t.z;
+    const double rho_d = safe_sqrt(r_d * r_d - J.rb * J.rb);
+    S.d = d;
+    S.inv_r = 1.0 / r_d;
+    S.rho = rho_d;
+    S.r = static_cast<float>(r_d);
+    S.c = static_cast<float>(J.rt * J.rt - r_d * r_d);
+    S.dmin = static_cast<float>(J.rt - r_d);
+    S.inv_range = static_cast<float>(1.0 / (rho_d + J.H - (J.rt - r_d)));
+    const double e = J.rb / r_d * J.sun_angular_radius;
+    S.e = static_cast<float>(e);
+    S.inv_span = static_cast<float>(0.5 / e);
+    const double ty = unit_to_texel(rho_d / J.H, J.th);
+    const Taps tt = axis_taps(ty, J.th);
+    S.t0 = tt.i0 * J.tw;
+    S.t1 = tt.i1 * J.tw;
+    S.wy = tt.w;
+    const double w = (tid == 0 || tid == kMarch - 1) ? 0.5 : 1.0;
+    const double dr = w * profile_density(J.prof_r, r_d - J.rb);
+    const double dm = w * profile_density(J.prof_m, r_d - J.rb);
+    for (int c = 0; c < 3; ++c) {
+      S.fr[c] = static_cast<float>(dr * tv[c]);
+      S.fm[c] = static_cast<float>(dm * tv[c]);
+    }
+  }
+  __syncthreads();
+
+  double mu_s[kTpt], nu[kTpt], rmus[kTpt];
+  bool on[kTpt];
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < kTpt; ++j) {
+    const int x = tile * kBlock * kTpt + j * kBlock + tid;
+    on[j] = x < W;
+    any = any || on[j];
+    mu_s[j] = on[j] ? s_col_mus(J, x % J.nmus) : 0.0;
+    nu[j] = on[j] ? s_slice_nu(J, x / J.nmus, mu, mu_s[j]) : 0.0;
+    rmus[j] = r * mu_s[j];
+  }
+  if (!any) return;
+  float ar[kTpt][3], am[kTpt][3];
+#pragma unroll
+  for (int j = 0; j < kTpt; ++j)
+    for (int c = 0; c < 3; ++c) ar[j][c] = am[j][c] = float(0);
+  for (int s = 0; s < kMarch; ++s) {
+    const SsFixedSample& S = smp[s];
+#pragma unroll
+    for (int j = 0; j < kTpt; ++j) {
+      if (!on[j]) continue;
+      const double t = fma(S.d, nu[j], rmus[j]);  // r * mu_s + d * nu = r_d * mu_s_d
+      const float xs = static_cast<float>((t + S.rho) * S.inv_r);  // mu_s_d - cos(theta_h)
+      // Clamps as max/min, 2 instructions each (the operands are finite; the
+      // ternary form, which also keeps NaNs, compiles to compares and
+      // selects).
+      const float mus = fmin(fmax(static_cast<float>(t * S.inv_r), float(-1)), float(1));
+      const float u = fmin(fmax((xs + S.e) * S.inv_span, float(0)), float(1));
+      const float vis = u * u * fma(float(-2), u, float(3));
+      float ts[3];
+      tsun_lookup(J, S, mus, ts);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float f = ts[c] * vis;
+        ar[j][c] = fma(f, S.fr[c], ar[j][c]);
+        am[j][c] = fma(f, S.fm[c], am[j][c]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kTpt; ++j) {
+    if (!on[j]) continue;
+    const int x = tile * kBlock * kTpt + j * kBlock + tid;
+    ss_store<false>(J, static_cast<int64_t>(row) * W + x, dx, ar[j], am[j]);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Scattering density (functions.glsl:1163-1260, :1348-1367).
 //
@@ -461,7 +614,7 @@ struct SdTheta {
 // mu_s; consecutive nu) of a thread. The phase function of the scattering
 // towards the view direction depends on (mu, theta_l, phi) only, so it is
 // computed once per azimuth pair for all kChunk outputs.
-template <int kChunk, bool kGround>
+template <int kChunk, bool kTwo, bool kGround>
 __device__ __forceinline__ void sd_theta(
     const float4* __restrict__ tab_a, const float4* __restrict__ tab_b,
     const float4* __restrict__ etab, float nu_max, float e_max, float A, float P,
@@ -507,32 +660,38 @@ __device__ __forceinline__ void sd_theta(
       for (int sgn = 0; sgn < 2; ++sgn) {
         const float t = sgn == 0 ? fmaf(tC[j], s, tb) : fmaf(-tC[j], s, tb);
         float3 v = table_lerp(tab_a, t);
-        // Order-1 incident radiance: Rayleigh and Mie single scattering
-        // times their phase functions of nu1 (constants folded in tables);
-        // x1 is the factor 1 + nu1^2 of both.
-        const float nu1 = fmaf(t, inv_hn, nu1_0);
-        const float3 vm = table_lerp(tab_b, t);
-        const float r1 = rsq_f(fmaf(mg2, nu1, g1));
-        const float q = r1 * r1 * r1;
-        const float x1 = fmaf(nu1, nu1, 1.0f);
-        v.x = fmaf(vm.x, q, v.x);
-        v.y = fmaf(vm.y, q, v.y);
-        v.z = fmaf(vm.z, q, v.z);
+        float x1 = 1.0f;
+        if (kTwo) {
+          // Order-1 incident radiance: Rayleigh and Mie single scattering
+          // times their phase functions of nu1 (constants folded in tables);
+          // x1 is the factor 1 + nu1^2 of both.
+          const float nu1 = fmaf(t, inv_hn, nu1_0);
+          const float3 vm = table_lerp(tab_b, t);
+          const float r1 = rsq_f(fmaf(mg2, nu1, g1));
+          const float q = r1 * r1 * r1;
+          x1 = fmaf(nu1, nu1, 1.0f);
+          v.x = fmaf(vm.x, q, v.x);
+          v.y = fmaf(vm.y, q, v.y);
+          v.z = fmaf(vm.z, q, v.z);
+        }
         if (kGround) {
-          v.x = x1 * v.x;
-          v.y = x1 * v.y;
-          v.z = x1 * v.z;
+          if (kTwo) {
+            v.x = x1 * v.x;
+            v.y = x1 * v.y;
+            v.z = x1 * v.z;
+          }
           const float3 e = table_lerp(etab, fmaf(eB, t, eA));
           v.x = fmaf(th.gf[0], e.x, v.x);
           v.y = fmaf(th.gf[1], e.y, v.y);
           v.z = fmaf(th.gf[2], e.z, v.z);
         }
         // l += x1 * v (with a ground term, x1 is in v).
+        constexpr bool kTimes = kTwo && !kGround;
         if (sgn == 0) {
-          l0 = kGround ? v.x : x1 * v.x;
-          l1 = kGround ? v.y : x1 * v.y;
-          l2 = kGround ? v.z : x1 * v.z;
-        } else if (!kGround) {
+          l0 = kTimes ? x1 * v.x : v.x;
+          l1 = kTimes ? x1 * v.y : v.y;
+          l2 = kTimes ? x1 * v.z : v.z;
+        } else if (kTimes) {
           l0 = fmaf(x1, v.x, l0);
           l1 = fmaf(x1, v.y, l1);
           l2 = fmaf(x1, v.z, l2);
@@ -555,7 +714,9 @@ __device__ __forceinline__ void sd_theta(
 //
 // kParts: threads that share an output, each summing kTheta / kParts of the
 // zenith angles (kSdSplit; 1 for the jobs that take none of it).
-template <int kChunk, int kB, int kParts>
+// kTwo: order 2; otherwise an order >= 3 of the models that do not take the arc
+// sums (fixed_sums), never in parts.
+template <int kChunk, int kB, int kParts, bool kTwo>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(5))) void
 k_scattering_density(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
@@ -594,7 +755,7 @@ k_scattering_density(
   const int stride = 2 * (nnu + 1);
   float4* tab_a = lds;
   float4* tab_b = lds + kTheta * stride;
-  float4* etab = lds + 2 * kTheta * stride;
+  float4* etab = lds + (kTwo ? 2 : 1) * kTheta * stride;
   const int tid = threadIdx.x;
 
   double r, rho;
@@ -632,8 +793,8 @@ k_scattering_density(
   }
   __syncthreads();
 
-  // Per-theta nu tables of the single scattering at (r, mu_s), mu rows
-  // blended, times d_omega and the phase-function constants.
+  // Per-theta nu tables of the order-(n-1) scattering at (r, mu_s), mu rows
+  // blended, times d_omega (and the phase-function constants for order 1).
   const float kR = static_cast<float>(3.0 / (16.0 * kPi));
   const double gd = J.g;
   const float kM = static_cast<float>(3.0 / (8.0 * kPi) * (1.0 - gd * gd) / (2.0 + gd * gd));
@@ -644,7 +805,7 @@ k_scattering_density(
     const int c0 = n * nmus + imus;
     const int c1 = (n + 1 < nnu ? n + 1 : n) * nmus + imus;
     const float wy = s_wy[l], wy0 = 1.0f - wy;
-    const float fa = s_dw[l] * kR;
+    const float fa = s_dw[l] * (kTwo ? kR : 1.0f);
     const float4* src = J.dR;
     float4 a0 = gload(src, r0 + c0), a1 = gload(src, r1 + c0);
     float4 b0 = gload(src, r0 + c1), b1 = gload(src, r1 + c1);
@@ -655,19 +816,21 @@ k_scattering_density(
     float4* ta = tab_a + l * stride;
     put_entry(ta, n + 1, v, vn);
     if (n == 0) put_entry(ta, 0, v, v);
-    const float fb = s_dw[l] * kM;
-    src = J.dM;
-    a0 = gload(src, r0 + c0);
-    a1 = gload(src, r1 + c0);
-    b0 = gload(src, r0 + c1);
-    b1 = gload(src, r1 + c1);
-    v = make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
-                    (wy0 * a0.z + wy * a1.z) * fb);
-    vn = make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
-                     (wy0 * b0.z + wy * b1.z) * fb);
-    float4* tb = tab_b + l * stride;
-    put_entry(tb, n + 1, v, vn);
-    if (n == 0) put_entry(tb, 0, v, v);
+    if (kTwo) {
+      const float fb = s_dw[l] * kM;
+      src = J.dM;
+      a0 = gload(src, r0 + c0);
+      a1 = gload(src, r1 + c0);
+      b0 = gload(src, r0 + c1);
+      b1 = gload(src, r1 + c1);
+      v = make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
+                      (wy0 * a0.z + wy * a1.z) * fb);
+      vn = make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
+                       (wy0 * b0.z + wy * b1.z) * fb);
+      float4* tb = tab_b + l * stride;
+      put_entry(tb, n + 1, v, vn);
+      if (n == 0) put_entry(tb, 0, v, v);
+    }
   }
   // Row 0 of delta irradiance (r = rb): the ground-irradiance lookup of the
   // reference at bottom_radius reads exactly this row.
@@ -733,10 +896,10 @@ k_scattering_density(
     const float4* tb = tab_b + l * stride;
     const bool g = __builtin_amdgcn_readfirstlane(t.ground) != 0;
     if (g)
-      sd_theta<kChunk, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+      sd_theta<kChunk, kTwo, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
                              acc);
     else
-      sd_theta<kChunk, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+      sd_theta<kChunk, kTwo, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
                               acc);
   }
   if (kParts > 1) {
@@ -1531,7 +1694,8 @@ int blocks_direct_irradiance(const Job& j) {
 int blocks_single_scattering(const Job& j) {
   const SsTiling t(j);
   if (t.nit == 0) return 0;  // served with its group's first
-  return (j.nnu * j.nmus + t.block - 1) / t.block * j.nmu * j.nr;
+  const int per_block = t.fixed ? kBlock * ss_texels_per_thread(j.nnu * j.nmus) : t.block;
+  return (j.nnu * j.nmus + per_block - 1) / per_block * j.nmu * j.nr;
 }
 int blocks_scattering_density(const Job& j) {
   const SdTile t = kSdTile[j.sd_tile];
@@ -1597,17 +1761,30 @@ void launch_ss_block(const PassLaunch& p, hipStream_t s) {
   launch_ss<true, 4, kB>(p, s);
   launch_ss<true, 5, kB>(p, s);
 }
+template <int kTpt>
+void launch_ss_fixed(const PassLaunch& p, hipStream_t s) {
+  if (kTpt < ss_texels_per_thread(p.min_w) || kTpt > ss_texels_per_thread(p.max_w)) return;
+  hipLaunchKernelGGL(k_single_scattering_fixed<kTpt>, dim3(p.total_blocks), dim3(kBlock), 0, s,
+                     p.jobs, p.first_block, p.njobs);
+}
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s) {
   // One instance per kind of job (SsTiling); each skips the others.
   launch_ss_block<64>(p, s);
   launch_ss_block<kBlock>(p, s);
   launch_ss_block<2 * kBlock>(p, s);
+  if (p.ss_kinds & kSsFixed) {
+    launch_ss_fixed<1>(p, s);
+    launch_ss_fixed<2>(p, s);
+    launch_ss_fixed<4>(p, s);
+  }
   return hipGetLastError();
 }
 template <int kChunk, int kB>
-void launch_sd_tile(const PassLaunch& p, size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL((k_scattering_density<kChunk, kB, 1>), dim3(p.total_blocks), dim3(kB), lds,
-                     s, p.jobs, p.first_block, p.njobs);
+void launch_sd_tile(const PassLaunch& p, int order, size_t lds, hipStream_t s) {
+  const auto kernel = order == 2 ? k_scattering_density<kChunk, kB, 1, true>
+                                 : k_scattering_density<kChunk, kB, 1, false>;
+  hipLaunchKernelGGL(kernel, dim3(p.total_blocks), dim3(kB), lds, s, p.jobs, p.first_block,
+                     p.njobs);
 }
 
 template <int kSplit>
@@ -1616,15 +1793,15 @@ void launch_sd_split(const PassLaunch& p, size_t lds, hipStream_t s) {
   static_assert(t.block / t.parts == 64, "a wave's outputs share their zenith angles");
   const size_t sums = sizeof(float) * 3 * t.chunk * t.block;
   if (p.sd_kinds & (1 << kSplit))
-    hipLaunchKernelGGL((k_scattering_density<t.chunk, t.block, t.parts>), dim3(p.total_blocks),
-                       dim3(t.block), lds > sums ? lds : sums, s, p.jobs, p.first_block,
-                       p.njobs);
+    hipLaunchKernelGGL((k_scattering_density<t.chunk, t.block, t.parts, true>),
+                       dim3(p.total_blocks), dim3(t.block), lds > sums ? lds : sums, s, p.jobs,
+                       p.first_block, p.njobs);
 }
 
-hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s) {
+hipError_t launch_scattering_density(const PassLaunch& p, int order, hipStream_t s) {
   // Tables of NU + 1 and E_W + 1 entries of two float4 (table_lerp).
   const size_t lds = sizeof(float4) *
-                     (static_cast<size_t>(4 * kTheta * (p.max_nnu + 1)) +
+                     (static_cast<size_t>((order == 2 ? 4 : 2) * kTheta * (p.max_nnu + 1)) +
                       2 * static_cast<size_t>(p.max_ew + 1));
   static_assert(kSdTiles == 6, "one case per tile shape");
   static_assert(kSdSplits == 3, "one launch per split");
@@ -1633,12 +1810,12 @@ hipError_t launch_scattering_density(const PassLaunch& p, hipStream_t s) {
   launch_sd_split<2>(p, lds, s);
   if ((p.sd_kinds & (1 << kSdSplits)) == 0) return hipGetLastError();
   switch (p.tile) {
-    case 0: launch_sd_tile<kSdTile[0].chunk, kSdTile[0].block>(p, lds, s); break;
-    case 1: launch_sd_tile<kSdTile[1].chunk, kSdTile[1].block>(p, lds, s); break;
-    case 2: launch_sd_tile<kSdTile[2].chunk, kSdTile[2].block>(p, lds, s); break;
-    case 3: launch_sd_tile<kSdTile[3].chunk, kSdTile[3].block>(p, lds, s); break;
-    case 4: launch_sd_tile<kSdTile[4].chunk, kSdTile[4].block>(p, lds, s); break;
-    case 5: launch_sd_tile<kSdTile[5].chunk, kSdTile[5].block>(p, lds, s); break;
+    case 0: launch_sd_tile<kSdTile[0].chunk, kSdTile[0].block>(p, order, lds, s); break;
+    case 1: launch_sd_tile<kSdTile[1].chunk, kSdTile[1].block>(p, order, lds, s); break;
+    case 2: launch_sd_tile<kSdTile[2].chunk, kSdTile[2].block>(p, order, lds, s); break;
+    case 3: launch_sd_tile<kSdTile[3].chunk, kSdTile[3].block>(p, order, lds, s); break;
+    case 4: launch_sd_tile<kSdTile[4].chunk, kSdTile[4].block>(p, order, lds, s); break;
+    case 5: launch_sd_tile<kSdTile[5].chunk, kSdTile[5].block>(p, order, lds, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

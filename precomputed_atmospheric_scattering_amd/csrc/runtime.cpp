@@ -628,8 +628,9 @@ atmo_status enqueue_precompute(atmo_model* m, unsigned orders, LaunchTimer& t) {
   for (unsigned order = 2; order <= orders; ++order) {
     const int o = static_cast<int>(order);
     ATMO_TRY(t.run(kSD, o, "scattering density", [&] {
-      return order == 2 ? atmo::launch_scattering_density(model_launch(m, 0, n, kSD), s)
-                        : atmo::launch_density_arcs(model_launch(m, 0, n, kSA), s);
+      return order == 2 || atmo::fixed_sums(m->jobs[0])
+                 ? atmo::launch_scattering_density(model_launch(m, 0, n, kSD), order, s)
+                 : atmo::launch_density_arcs(model_launch(m, 0, n, kSA), s);
     }));
     ATMO_TRY(t.run(kII, o - 1, "indirect irradiance", [&] {
       return atmo::launch_indirect_irradiance(model_launch(m, 0, n, kII), o - 1, s);
@@ -1526,7 +1527,11 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     std::vector<std::pair<int, int>> on;
     for (const auto& mj : sel)
       if (orders[mj.first] >= n) on.push_back(mj);
-    add_level(n == 2 ? kSD : kSA, static_cast<int>(n), on);
+    std::vector<std::pair<int, int>> direct, arcs;
+    for (const auto& mj : on)
+      (n == 2 || atmo::fixed_sums(models[mj.first]->jobs[0]) ? direct : arcs).push_back(mj);
+    add_level(kSD, static_cast<int>(n), direct);
+    add_level(kSA, static_cast<int>(n), arcs);
     add_level(kII, static_cast<int>(n) - 1, on);
     add_level(kMS, 0, on);
   }
@@ -1591,7 +1596,7 @@ atmo_status launch_level(const Level& l, const atmo::Job* d_jobs, const int* d_f
     case kT: e = atmo::launch_transmittance(pl, s); break;
     case kE0: e = atmo::launch_direct_irradiance(pl, s); break;
     case kSS: e = atmo::launch_single_scattering(pl, s); break;
-    case kSD: e = atmo::launch_scattering_density(pl, s); break;
+    case kSD: e = atmo::launch_scattering_density(pl, l.order, s); break;
     case kSA: e = atmo::launch_density_arcs(pl, s); break;
     case kII: e = atmo::launch_indirect_irradiance(pl, l.order, s); break;
     case kMS: e = atmo::launch_multiple_scattering(pl, s); break;

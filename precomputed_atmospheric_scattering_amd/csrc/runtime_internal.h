@@ -37,7 +37,7 @@ struct Sizes {
 };
 
 
-// kSD: scattering density of order 2; kSA: of the orders >= 3.
+// kSD: scattering density direction by direction; kSA: by arc sums (orders >= 3).
 enum Pass { kT = 0, kE0, kSS, kSD, kII, kMS, kAcc, kHalf, kClear, kPack, kOD, kSA, kPasses };
 
 
