@@ -208,6 +208,12 @@ ATMO_HD int ms_rows_per_block(int w, int capacity) {
   const int cap = capacity <= kBlock ? 4 : 8;
   return r < cap ? r : cap;
 }
+// Rows per block of a tile of tpt texels per thread, whose texels are in one row
+// (odd rows of two-texel tiles leave a thread's second texel idle).
+ATMO_HD int ms_tile_rows(int w, int tpt, int block) {
+  const int r = ms_rows_per_block(w, tpt * block), m = block / ((w + tpt - 1) / tpt);
+  return r < m ? r : m;
+}
 // The smallest tile that holds a row of w texels.
 ATMO_HD int ms_default_tile(int w) {
   if (w <= kBlock) return 0;

@@ -1067,9 +1067,15 @@ __global__ __launch_bounds__(64) void k_indirect_irradiance(
 // one row in LDS with coalesced loads (every texel of a row reads the same
 // four rows), and each texel then reads its 4 (mu_s, nu) taps from LDS:
 // 4 coalesced global loads per texel and sample instead of 16 gathers.
-// Each of the kB threads holds kTpt texels; a block takes
-// ms_rows_per_block(W, kTpt * kB) whole rows (several short rows, or one row
-// of up to kTpt * kB texels). Rows longer than kMsMaxRow take the per-texel 16-tap gather of
+// Each of the kB threads holds kTpt texels of one row, whose samples it reads
+// once; a block takes ms_tile_rows whole rows (several short rows, or one row
+// of up to kTpt * kB texels). FP16 models' threads load two neighbouring texels
+// at a time: at rows of 1024 texels and 15 wavelengths 75.5 ms per Init of 8
+// orders against 81.0 with a load per texel and the samples read for each (the
+// address units busy 45% of the time instead of 65%; then the LDS is, 81%); at
+// rows of 256, 1.90 ms against 1.97 (4 orders); FP32 rows of 1024 with 3
+// wavelengths 6.30 against 6.41. (16 bytes per texel in LDS, for 16-byte reads,
+// took 10-20% more.) Rows longer than kMsMaxRow take the per-texel 16-tap gather of
 // k_multiple_scattering_gather. Both kernels are launched over the same
 // blocks and each returns at once on the other's jobs, so the path of a job
 // depends on its own row length only.
@@ -1135,6 +1141,20 @@ struct MsRowSample {
   float pad;
 };
 
+// A load of delta J at a byte offset: 12 bytes, or two 8-byte texels.
+template <class T>
+__device__ __forceinline__ T ms_load(const char* __restrict__ D, uint32_t at);
+template <>
+__device__ __forceinline__ float3 ms_load<float3>(const char* __restrict__ D, uint32_t at) {
+  return gload_at(reinterpret_cast<const float3*>(D), at);
+}
+template <>
+__device__ __forceinline__ uint4 ms_load<uint4>(const char* __restrict__ D, uint32_t at) {
+  typedef uint32_t Pair __attribute__((ext_vector_type(4), aligned(8)));
+  const Pair v = gload_at(reinterpret_cast<const Pair*>(D), at);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // kF16: the kernel serves the jobs whose delta J is 3 x 21-bit floats
 // (FP16-storage models); otherwise the FP32 ones. Both are launched over the
 // same blocks when a launch holds both kinds; each returns at once on the
@@ -1146,7 +1166,6 @@ template <int kTpt, bool kF16, int kB>
 __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
     int njobs, int max_rows) {
-  using Src = typename std::conditional<kF16, uint2, float3>::type;
   // Dynamic LDS: two buffers of kB * kTpt blended texels, then the
   // samples of max_rows rows (the launch's largest rows per block).
   // Blended texels are RGB (12 bytes), so that more blocks fit a CU's LDS.
@@ -1160,7 +1179,7 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   const int lb = blockIdx.x - first_block[ji];
   const int nnu = J.nnu, nmus = J.nmus, nmu = J.nmu;
   const int W = nnu * nmus;
-  const int rpb = ms_rows_per_block(W, kTpt * kB);
+  const int rpb = ms_tile_rows(W, kTpt, kB);
   // Gather-path job (uniform per block). The launcher groups jobs by tile
   // and sizes max_rows over them; the tests only keep LDS indexing in
   // bounds should it not.
@@ -1192,7 +1211,7 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
     MsRowSample& S = smp[slot][i];
     S.d = d;
     S.inv_r = 1.0 / r_i;
-    const uint32_t row_bytes = static_cast<uint32_t>(W) * sizeof(Src);
+    const uint32_t row_bytes = static_cast<uint32_t>(W) * (kF16 ? 8u : 12u);
     S.o00 = static_cast<uint32_t>(tz.i0 * nmu + ty.i0) * row_bytes;
     S.o01 = static_cast<uint32_t>(tz.i0 * nmu + ty.i1) * row_bytes;
     S.o10 = static_cast<uint32_t>(tz.i1 * nmu + ty.i0) * row_bytes;
@@ -1211,22 +1230,24 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   // functions.glsl:967-973) and r mu_s.
   // c0_of, c1_of: LDS byte offsets of the texel's two nu slices in a
   // blended row (the slice's first texel).
-  int slot_of[kTpt], x_of[kTpt];
+  // The texels of a thread are in one row, x and x + tpr: its samples are read
+  // once.
+  const int tpr = (W + kTpt - 1) / kTpt;  // threads per row
+  const int slot = tid / tpr < rpb && row0 + tid / tpr < nrows ? tid / tpr : -1;
+  int x_of[kTpt];  // or -1
   uint32_t c0_of[kTpt], c1_of[kTpt];
   float ws_of[kTpt];
   double nu_of[kTpt], rmus_of[kTpt];
   float acc[kTpt][3];
 #pragma unroll
   for (int j = 0; j < kTpt; ++j) {
-    const int f = tid + j * kB;
-    const int slot = f / W;
-    slot_of[j] = (slot < rpb && row0 + slot < nrows) ? slot : -1;
-    x_of[j] = f - slot * W;
+    x_of[j] = tid - tid / tpr * tpr + j * tpr;
+    if (slot < 0 || x_of[j] >= W) x_of[j] = -1;
     acc[j][0] = acc[j][1] = acc[j][2] = 0.0f;
     c0_of[j] = c1_of[j] = 0u;
     ws_of[j] = 0.0f;
     nu_of[j] = rmus_of[j] = 0.0;
-    if (slot_of[j] < 0) continue;
+    if (x_of[j] < 0) continue;
     const int2 zy = ms_row(J, row0 + slot);
     const int z = zy.x, y = zy.y;
     double r, rho, mu;
@@ -1253,66 +1274,78 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   __syncthreads();
 
   const MusMap mus_map(J);
-  const Src* __restrict__ D = static_cast<const Src*>(J.dJ);
-  uint32_t x_bytes[kTpt];
+  // What a thread blends. FP32: its texels. FP16: two neighbours, with 16-byte
+  // loads (a load of 64 lanes costs 16 cycles at 8, 12 or 16 bytes a lane);
+  // the last pair of an odd row overlaps the one before it. With one texel per
+  // thread, half of the waves blend.
+  constexpr int kLoads = kF16 ? 1 : kTpt;
+  using Load = typename std::conditional<kF16, uint4, float3>::type;
+  const int ppr = kF16 ? (W + 1) / 2 : tpr;  // threads that blend per row
+  const int from = kTpt == 1 && kF16
+                       ? (tid / ppr < rpb && row0 + tid / ppr < nrows ? tid / ppr : -1)
+                       : slot;
+  const MsRowSample* const blend = smp[from < 0 ? 0 : from];
+  const MsRowSample* const march = smp[slot < 0 ? 0 : slot];
+  const int pair = kF16 ? min(2 * (tid - tid / ppr * ppr), W - 2) : 0;
+  uint32_t x_bytes[kLoads], to[kLoads];  // in a source row; in a buffer
 #pragma unroll
-  for (int j = 0; j < kTpt; ++j)
-    x_bytes[j] = static_cast<uint32_t>(x_of[j]) * static_cast<uint32_t>(sizeof(Src));
+  for (int j = 0; j < kLoads; ++j) {
+    const int x = kF16 ? pair : (x_of[j] < 0 ? 0 : x_of[j]);
+    x_bytes[j] = static_cast<uint32_t>(x) * static_cast<uint32_t>(kF16 ? 8 : 12);
+    to[j] = static_cast<uint32_t>((from < 0 ? 0 : from) * W + x);
+  }
+  const char* __restrict__ D = static_cast<const char*>(J.dJ);
   // Source texels of the next sample, loaded one sample ahead so that the
   // loads are in flight during the barrier and the gather of the current one.
-  Src src[kTpt][4];
+  Load src[kLoads][4];
   auto fetch = [&](int i) {
+    // FP32: idle lanes load row slot 0's texel 0, in bounds, so that the loads
+    // need no branch.
+    if (kF16 && from < 0) return;
+    const MsRowSample& S = blend[i];
 #pragma unroll
-    for (int j = 0; j < kTpt; ++j) {
-      // Idle lanes (slot -1) load row slot 0's texel 0, in bounds, so that
-      // the loads need no branch.
-      const bool on = slot_of[j] >= 0;
-      const MsRowSample& S = smp[on ? slot_of[j] : 0][i];
-      const uint32_t xb = on ? x_bytes[j] : 0u;
-      src[j][0] = gload_at(D, S.o00 + xb);
-      src[j][1] = gload_at(D, S.o01 + xb);
-      src[j][2] = gload_at(D, S.o10 + xb);
-      src[j][3] = gload_at(D, S.o11 + xb);
+    for (int j = 0; j < kLoads; ++j) {
+      src[j][0] = ms_load<Load>(D, S.o00 + x_bytes[j]);
+      src[j][1] = ms_load<Load>(D, S.o01 + x_bytes[j]);
+      src[j][2] = ms_load<Load>(D, S.o10 + x_bytes[j]);
+      src[j][3] = ms_load<Load>(D, S.o11 + x_bytes[j]);
     }
   };
   fetch(0);
   for (int i = 0; i < kMarch; ++i) {
     float3* B = buf + (i & 1) * (kB * kTpt);
     // Blend the four (r, mu) source rows of sample i into LDS.
-#pragma unroll
-    for (int j = 0; j < kTpt; ++j) {
-      if (slot_of[j] < 0) continue;
-      const MsRowSample& S = smp[slot_of[j]][i];
-      float3 a, b, c, e;
+    if (from >= 0) {
+      const MsRowSample& S = blend[i];
       const float w00 = S.w00, w01 = S.w01, w10 = S.w10, w11 = S.w11;
-      if (kF16) {
-        const uint2* u = reinterpret_cast<const uint2*>(src[j]);
-        a = unpack_f21x3(u[0]);
-        b = unpack_f21x3(u[1]);
-        c = unpack_f21x3(u[2]);
-        e = unpack_f21x3(u[3]);
-      } else {
-        const float3* f = reinterpret_cast<const float3*>(src[j]);
-        a = f[0];
-        b = f[1];
-        c = f[2];
-        e = f[3];
+      auto mix = [&](float3 a, float3 b, float3 c, float3 e) {
+        return make_float3(fmaf(w11, e.x, fmaf(w10, c.x, fmaf(w01, b.x, w00 * a.x))),
+                           fmaf(w11, e.y, fmaf(w10, c.y, fmaf(w01, b.y, w00 * a.y))),
+                           fmaf(w11, e.z, fmaf(w10, c.z, fmaf(w01, b.z, w00 * a.z))));
+      };
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        if constexpr (kF16) {
+          auto half = [&](int k, int c) {
+            return unpack_f21x3(c == 0 ? make_uint2(src[j][k].x, src[j][k].y)
+                                       : make_uint2(src[j][k].z, src[j][k].w));
+          };
+          B[to[j]] = mix(half(0, 0), half(1, 0), half(2, 0), half(3, 0));
+          B[to[j] + 1] = mix(half(0, 1), half(1, 1), half(2, 1), half(3, 1));
+        } else if (x_of[j] >= 0) {
+          B[to[j]] = mix(src[j][0], src[j][1], src[j][2], src[j][3]);
+        }
       }
-      float3 v;
-      v.x = fmaf(w11, e.x, fmaf(w10, c.x, fmaf(w01, b.x, w00 * a.x)));
-      v.y = fmaf(w11, e.y, fmaf(w10, c.y, fmaf(w01, b.y, w00 * a.y)));
-      v.z = fmaf(w11, e.z, fmaf(w10, c.z, fmaf(w01, b.z, w00 * a.z)));
-      B[tid + j * kB] = v;
     }
     if (i + 1 < kMarch) fetch(i + 1);
     // One barrier per sample: buffer i & 1 is written again at sample i + 2,
     // after every thread has passed the barrier of sample i + 1 and so has
     // finished reading it.
     __syncthreads();
+    const MsRowSample& S = march[i];
 #pragma unroll
     for (int j = 0; j < kTpt; ++j) {
-      if (slot_of[j] < 0) continue;
-      const MsRowSample& S = smp[slot_of[j]][i];
+      if (x_of[j] < 0) continue;
       // mu_s at the sample, (r mu_s + d nu) / r_i (functions.glsl:1311).
       const float mus =
           clampf(static_cast<float>(fma(S.d, nu_of[j], rmus_of[j]) * S.inv_r), -1.0f, 1.0f);
@@ -1340,8 +1373,8 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
 
 #pragma unroll
   for (int j = 0; j < kTpt; ++j) {
-    if (slot_of[j] < 0) continue;
-    const int2 zy = ms_row(J, row0 + slot_of[j]);
+    if (x_of[j] < 0) continue;
+    const int2 zy = ms_row(J, row0 + slot);
     const int z = zy.x, y = zy.y;
     const int64_t t_idx = (static_cast<int64_t>(z) * nmu + y) * W + x_of[j];
     gstore(J.dR, t_idx, make_float4(acc[j][0], acc[j][1], acc[j][2], 0.0f));
@@ -1709,7 +1742,7 @@ int blocks_scattering_density(const Job& j) {
 int blocks_indirect_irradiance(const Job& j) { return j.ew * j.eh; }
 int blocks_multiple_scattering(const Job& j) {
   const int w = j.nnu * j.nmus;
-  const int rpb = ms_rows_per_block(w, ms_tile_capacity(j.ms_tile));
+  const int rpb = ms_tile_rows(w, kMsTile[j.ms_tile].tpt, kMsTile[j.ms_tile].block);
   const int rows = j.nmu * j.nr;
   if (rpb == 0) return ((w + kBlock - 1) / kBlock) * rows;
   if (rpb < 0) return 0;  // not a tile of this row length (rejected by the host)
