@@ -603,6 +603,31 @@ __device__ __forceinline__ void put_entry(float4* tab, int k, float3 v, float3 v
   tab[2 * k + 1] = make_float4(vn.y - v.y, vn.z - v.z, 0.f, 0.f);
 }
 
+// Order 2 interpolates two tables at the same coordinate: entries of three
+// float4 hold (v, dv) of both, (a.x, a.y, a.z, da.x), (da.y, da.z, b.x, b.y),
+// (b.z, db.x, db.y, db.z): one address and three loads where two tables of two
+// float4 took two and four. The pass is bound by vector instructions, then LDS:
+// .419 ms against .438 (1.05M texels, 3 wavelengths), 25.5 against 26.2 (16.8M,
+// 15), .497 against .547 (.39M, 9).
+struct TwoLerp {
+  float3 a, b;
+};
+__device__ __forceinline__ TwoLerp table_lerp2(const float4* __restrict__ tab, float t1) {
+  float w;
+  const int i = split_coord(t1, &w);
+  const float4* const e = reinterpret_cast<const float4*>(
+      reinterpret_cast<const char*>(tab) + __umul24(static_cast<uint32_t>(i), 48u));
+  const float4 e0 = e[0], e1 = e[1], e2 = e[2];
+  return {make_float3(fmaf(w, e0.w, e0.x), fmaf(w, e1.x, e0.y), fmaf(w, e1.y, e0.z)),
+          make_float3(fmaf(w, e2.y, e1.z), fmaf(w, e2.z, e1.w), fmaf(w, e2.w, e2.x))};
+}
+__device__ __forceinline__ void put_entry2(float4* tab, int k, float3 a, float3 an, float3 b,
+                                           float3 bn) {
+  tab[3 * k] = make_float4(a.x, a.y, a.z, an.x - a.x);
+  tab[3 * k + 1] = make_float4(an.y - a.y, an.z - a.z, b.x, b.y);
+  tab[3 * k + 2] = make_float4(b.z, bn.x - b.x, bn.y - b.y, bn.z - b.z);
+}
+
 struct SdTheta {
   float cos_t, sin_t;
   float ga, gb;   // ground normal . sun = ga + gb * nu1
@@ -616,8 +641,8 @@ struct SdTheta {
 // computed once per azimuth pair for all kChunk outputs.
 template <int kChunk, bool kTwo, bool kGround>
 __device__ __forceinline__ void sd_theta(
-    const float4* __restrict__ tab_a, const float4* __restrict__ tab_b,
-    const float4* __restrict__ etab, float nu_max, float e_max, float A, float P,
+    const float4* __restrict__ tab, const float4* __restrict__ etab, float nu_max,
+    float e_max, float A, float P,
     float Q, const float (&Bv)[kChunk], const float (&Cv)[kChunk], float g1,
     float mg2, const float cR[3], const float cM[3], const SdTheta& th,
     float (&acc)[kChunk][3]) {
@@ -659,14 +684,18 @@ __device__ __forceinline__ void sd_theta(
 #pragma unroll
       for (int sgn = 0; sgn < 2; ++sgn) {
         const float t = sgn == 0 ? fmaf(tC[j], s, tb) : fmaf(-tC[j], s, tb);
-        float3 v = table_lerp(tab_a, t);
+        float3 v;
         float x1 = 1.0f;
-        if (kTwo) {
+        if (!kTwo) {
+          v = table_lerp(tab, t);
+        } else {
           // Order-1 incident radiance: Rayleigh and Mie single scattering
           // times their phase functions of nu1 (constants folded in tables);
           // x1 is the factor 1 + nu1^2 of both.
           const float nu1 = fmaf(t, inv_hn, nu1_0);
-          const float3 vm = table_lerp(tab_b, t);
+          const TwoLerp both = table_lerp2(tab, t);
+          const float3 vm = both.b;
+          v = both.a;
           const float r1 = rsq_f(fmaf(mg2, nu1, g1));
           const float q = r1 * r1 * r1;
           x1 = fmaf(nu1, nu1, 1.0f);
@@ -752,10 +781,9 @@ k_scattering_density(
   const int W = nnu * nmus;
   // Per theta a table of NU + 1 entries (table_lerp); then the
   // ground-irradiance table of E_W + 1 entries.
-  const int stride = 2 * (nnu + 1);
-  float4* tab_a = lds;
-  float4* tab_b = lds + kTheta * stride;
-  float4* etab = lds + (kTwo ? 2 : 1) * kTheta * stride;
+  const int stride = (kTwo ? 3 : 2) * (nnu + 1);
+  float4* tab = lds;
+  float4* etab = lds + kTheta * stride;
   const int tid = threadIdx.x;
 
   double r, rho;
@@ -813,23 +841,25 @@ k_scattering_density(
                            (wy0 * a0.z + wy * a1.z) * fa);
     float3 vn = make_float3((wy0 * b0.x + wy * b1.x) * fa, (wy0 * b0.y + wy * b1.y) * fa,
                             (wy0 * b0.z + wy * b1.z) * fa);
-    float4* ta = tab_a + l * stride;
-    put_entry(ta, n + 1, v, vn);
-    if (n == 0) put_entry(ta, 0, v, v);
-    if (kTwo) {
+    float4* ta = tab + l * stride;
+    if (!kTwo) {
+      put_entry(ta, n + 1, v, vn);
+      if (n == 0) put_entry(ta, 0, v, v);
+    } else {
       const float fb = s_dw[l] * kM;
       src = J.dM;
       a0 = gload(src, r0 + c0);
       a1 = gload(src, r1 + c0);
       b0 = gload(src, r0 + c1);
       b1 = gload(src, r1 + c1);
-      v = make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
+      const float3 m =
+          make_float3((wy0 * a0.x + wy * a1.x) * fb, (wy0 * a0.y + wy * a1.y) * fb,
                       (wy0 * a0.z + wy * a1.z) * fb);
-      vn = make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
-                       (wy0 * b0.z + wy * b1.z) * fb);
-      float4* tb = tab_b + l * stride;
-      put_entry(tb, n + 1, v, vn);
-      if (n == 0) put_entry(tb, 0, v, v);
+      const float3 mn =
+          make_float3((wy0 * b0.x + wy * b1.x) * fb, (wy0 * b0.y + wy * b1.y) * fb,
+                      (wy0 * b0.z + wy * b1.z) * fb);
+      put_entry2(ta, n + 1, v, vn, m, mn);
+      if (n == 0) put_entry2(ta, 0, v, v, m, m);
     }
   }
   // Row 0 of delta irradiance (r = rb): the ground-irradiance lookup of the
@@ -892,14 +922,13 @@ k_scattering_density(
       Bv[jn] = fsx[jn] * t.sin_t;
       Cv[jn] = fsy[jn] * t.sin_t;
     }
-    const float4* ta = tab_a + l * stride;
-    const float4* tb = tab_b + l * stride;
+    const float4* ta = tab + l * stride;
     const bool g = __builtin_amdgcn_readfirstlane(t.ground) != 0;
     if (g)
-      sd_theta<kChunk, kTwo, true>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+      sd_theta<kChunk, kTwo, true>(ta, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
                              acc);
     else
-      sd_theta<kChunk, kTwo, false>(ta, tb, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
+      sd_theta<kChunk, kTwo, false>(ta, etab, nu_max, e_max, A, P, Q, Bv, Cv, g1, mg2, cR, cM, t,
                               acc);
   }
   if (kParts > 1) {
@@ -1832,9 +1861,9 @@ void launch_sd_split(const PassLaunch& p, size_t lds, hipStream_t s) {
 }
 
 hipError_t launch_scattering_density(const PassLaunch& p, int order, hipStream_t s) {
-  // Tables of NU + 1 and E_W + 1 entries of two float4 (table_lerp).
+  // Tables of NU + 1 and E_W + 1 entries (table_lerp2, table_lerp).
   const size_t lds = sizeof(float4) *
-                     (static_cast<size_t>((order == 2 ? 4 : 2) * kTheta * (p.max_nnu + 1)) +
+                     (static_cast<size_t>((order == 2 ? 3 : 2) * kTheta * (p.max_nnu + 1)) +
                       2 * static_cast<size_t>(p.max_ew + 1));
   static_assert(kSdTiles == 6, "one case per tile shape");
   static_assert(kSdSplits == 3, "one launch per split");
