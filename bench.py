@@ -86,11 +86,19 @@ PROFILES = os.path.join(ROOT, "profiles")
 COUNTERS_HIGH_RES = os.path.join(PROFILES, "counters_high_resolution.md")
 VALU_MIX_HIGH_RES = os.path.join(PROFILES, "valu_mix_high_resolution.md")
 # Pass -> kernel of the counter summary (the transmittance pass's launches
-# are two kernels, the optical depths and the LUT, and carry no counters).
-PASS_KERNELS = dict(single_scattering="k_single_scattering",
-                    scattering_density="k_scattering_density",
-                    indirect_irradiance="k_indirect_irradiance",
-                    multiple_scattering="k_multiple_scattering")
+# are two kernels, the optical depths and the LUT, and carry no counters). The
+# density is one kernel at order 2 and another at the orders >= 3.
+PASS_KERNELS = dict(single_scattering=("k_single_scattering",),
+                    scattering_density=("k_scattering_density", "k_density_arcs"),
+                    indirect_irradiance=("k_indirect_irradiance",),
+                    multiple_scattering=("k_multiple_scattering",))
+
+
+def launch_kernel(name):
+    """Kernel of a launch, by its name ('scattering_density_2' and others)."""
+    if name.startswith("scattering_density"):
+        return PASS_KERNELS["scattering_density"][0 if name.endswith("_2") else 1]
+    return PASS_KERNELS.get(name, ("",))[0]
 
 
 def percentile(xs, q):
@@ -632,24 +640,33 @@ def pass_figures(launches, steps, n_s, iters):
     its MI355X peak."""
     cnt = counter_figures()
     mix = valu_mix_figures()
-    merged = {}
+    merged, kernels = {}, {}
     for k, v in launches.items():
-        merged.setdefault("scattering_density" if k.startswith("scattering_density") else k,
-                          []).extend(v)
+        name = "scattering_density" if k.startswith("scattering_density") else k
+        merged.setdefault(name, []).extend(v)
+        kernels.setdefault(name, []).extend([launch_kernel(k)] * len(v))
+
+    def per_launch(table, name, pick):
+        """Average over a pass's launches of a figure of their kernels, or None."""
+        if not all(k in table for k in kernels[name]):
+            return None
+        return sum(pick(table[k]) for k in kernels[name]) / len(kernels[name])
+
     out = {}
     for name, ms_list in merged.items():
         avg_s = sum(ms_list) / len(ms_list) * 1e-3
         e = {"ms_per_atmosphere": round(sum(ms_list) / steps, 3),
              "launches_per_atmosphere": len(ms_list) // steps,
              "avg_launch_ms": round(avg_s * 1e3, 4)}
-        c = cnt.get(PASS_KERNELS.get(name, ""))
-        if c is not None:
-            e["valu_tops"] = round(c["valu"] * 64.0 / avg_s / 1e12, 3)
-            e["valu_frac"] = round(c["valu"] * 64.0 / avg_s / 1e12 / PEAK_VALU_TOPS, 4)
-            e["hbm_bytes_per_launch"] = round(c["fetch"] + c["write"])
-            e["hbm_gb_per_s"] = round((c["fetch"] + c["write"]) / avg_s / 1e9, 1)
-            e["hbm_frac"] = round((c["fetch"] + c["write"]) / avg_s / 1e9 / PEAK_HBM_GBS, 4)
-        fa = mix.get(PASS_KERNELS.get(name, ""))
+        valu = per_launch(cnt, name, lambda c: c["valu"])
+        if valu is not None:
+            hbm = per_launch(cnt, name, lambda c: c["fetch"] + c["write"])
+            e["valu_tops"] = round(valu * 64.0 / avg_s / 1e12, 3)
+            e["valu_frac"] = round(valu * 64.0 / avg_s / 1e12 / PEAK_VALU_TOPS, 4)
+            e["hbm_bytes_per_launch"] = round(hbm)
+            e["hbm_gb_per_s"] = round(hbm / avg_s / 1e9, 1)
+            e["hbm_frac"] = round(hbm / avg_s / 1e9 / PEAK_HBM_GBS, 4)
+        fa = per_launch(mix, name, lambda v: v)
         if fa is not None:
             e["fp_arith_tops"] = round(fa * 64.0 / avg_s / 1e12, 3)
             e["fp_arith_frac"] = round(fa * 64.0 / avg_s / 1e12 / PEAK_FP_ARITH_TOPS, 4)
@@ -691,7 +708,7 @@ def roofline(passes):
             "frac": p["fp_arith_frac"],
             "counters": os.path.relpath(VALU_MIX_HIGH_RES, ROOT)}}
     return dict({
-        "kernel": PASS_KERNELS[name],
+        "kernel": " + ".join(PASS_KERNELS[name]),
         "bound": "valu" if valu else "hbm",
         "achieved": p["valu_tops"] if valu else p["hbm_gb_per_s"],
         "peak": round(PEAK_VALU_TOPS, 2) if valu else PEAK_HBM_GBS,

@@ -384,12 +384,22 @@ ATMO_HD double s_r_texel(const Job& j, double r) {
   return unit_to_texel(rho / j.H, j.nr);
 }
 
+// rb^2 as a rounded product, never part of a fused multiply-add: where a ray
+// grazes the ground, the discriminant below and rho^2 are differences of nearly
+// equal squares, and a lookup moves by percents if only one of them is rounded.
+ATMO_HD double rb_squared(const Job& j) {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+  return j.rb * j.rb;
+}
+
 // functions.glsl:789-812 (u_mu), as GL texel-space y. The ground and sky
 // halves each map to MU/2 texels.
 ATMO_HD double s_mu_texel(const Job& j, double r, double mu, bool ground) {
   double rho = safe_sqrt(r * r - j.rb * j.rb);
   double r_mu = r * mu;
-  double disc = r_mu * r_mu - r * r + j.rb * j.rb;
+  double disc = r_mu * r_mu - r * r + rb_squared(j);
   const int half = j.nmu / 2;
   double u_mu;
   if (ground) {
