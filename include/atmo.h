@@ -235,11 +235,14 @@ int atmo_batch_num_launches(const atmo_batch* batch);
 void atmo_batch_destroy(atmo_batch* batch);
 
 /* Tile shapes and their autotuner (no counterpart in the reference, whose
- * passes are fragment-shader draws). The scattering-density pass runs with
- * sd_nu_per_thread nu outputs per thread in blocks of sd_block_threads; the
- * multiple-scattering pass with ms_texels_per_thread texels per thread in
- * blocks of ms_block_threads, its blocks walking the (r, mu) rows of the LUT r-major (ms_row_order 0, the
- * LUT's own order), mu-major (1) or in ray order (2: rows sorted by the
+ * passes are fragment-shader draws). The scattering density, where it is
+ * summed direction by direction with a thread per output (order 2 of LUTs of
+ * more than 1.25M texels times Precompute iterations; every order of
+ * half-precision models of up to 2^22 texels), runs with sd_nu_per_thread nu
+ * outputs per thread in blocks of sd_block_threads. The multiple-scattering
+ * pass runs with ms_texels_per_thread texels per thread in blocks of
+ * ms_block_threads, its blocks walking the (r, mu) rows of the LUT r-major
+ * (ms_row_order 0, the LUT's own order), mu-major (1) or in ray order (2: rows sorted by the
  * impact parameter r sqrt(1 - mu^2) of their view ray, so that blocks that
  * run together read the same source rows).
  * Every shape computes each texel identically: the LUTs do not depend on

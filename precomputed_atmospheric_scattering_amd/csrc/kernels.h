@@ -44,7 +44,7 @@ constexpr int kBlock = 256;
 // with the same operations in the same order, so the LUTs do not depend on
 // the choice.
 //
-// Scattering density of order 2: nu outputs per thread (they share the phase
+// Scattering density direction by direction: nu outputs per thread (they share the phase
 // function of the outgoing direction) and threads per block. A (r, mu_s) plane of
 // MU x ceil(NU / chunk) threads is split into ceil(plane / block) blocks,
 // each of which builds the plane's nu tables in LDS.
