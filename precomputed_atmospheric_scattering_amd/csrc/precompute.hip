@@ -963,20 +963,25 @@ k_scattering_density(
 
 // ---------------------------------------------------------------------------
 // Indirect irradiance (functions.glsl:1477-1511, :1573-1586) and the packing
-// of atmosphere/model.cc:176-190. One wave per irradiance texel: the wave
-// builds, for each of the 16 zenith angles, the nu table of the scattering at
-// (r, mu = cos theta, mu_s) (trilinear in r, mu, mu_s), then each lane takes
-// one of the 64 azimuths, sums over theta, and the wave reduces. One wave per
-// block, so the tables of a texel need at most 4 * 16 * (NU + 1) float4 of
-// LDS (table_lerp's layout).
+// of atmosphere/model.cc:176-190. One block per irradiance texel: it builds, for
+// each of the 16 zenith angles, the nu table of the scattering at (r, mu = cos
+// theta, mu_s) (trilinear in r, mu, mu_s), an entry per thread, from LDS
+// constants of the angles; then each lane of the first wave takes one of the 64
+// azimuths, sums over theta, and the wave reduces. The pass is a chain of
+// latencies: with one wave building the tables, each lane computing the sines
+// and mu coordinates of its entries and of all angles again, a launch took 14.5
+// us (128 texels), now 9.8; per Init of 4 orders at 64 x 16 texels .063 ms against
+// .041 (3 wavelengths) and .141 against .107 (15). The tables of a texel need at
+// most 4 * 16 * (NU + 1) float4 of LDS (table_lerp's layout).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_indirect_irradiance(
+constexpr int kIiBlock = 256;
+__global__ __launch_bounds__(kIiBlock) void k_indirect_irradiance(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
     int njobs, int order) {
   extern __shared__ float4 lds[];
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int texel = blockIdx.x - first_block[ji];
   const int nnu = J.nnu, nmus = J.nmus, nmu = J.nmu;
   const bool one = order == 1;
@@ -989,53 +994,67 @@ __global__ __launch_bounds__(64) void k_indirect_irradiance(
   if (active) e_rmus_from_texel(J, texel % J.ew, texel / J.ew, &r, &mu_s);
   const int W = nnu * nmus;
   const double dtheta = kPi / 32.0, dphi = kPi / 32.0;
+  // What depends on the zenith angle.
+  __shared__ struct {
+    float fct, fst, f, wy;
+    int y0, y1;
+  } th[kTheta];
+  if (tid < kTheta) {
+    const double theta = (tid + 0.5) * dtheta;
+    const double ct = cos(theta), st = sin(theta);
+    const Taps ty = axis_taps(s_mu_texel(J, r, ct, false), nmu);
+    th[tid].fct = static_cast<float>(ct);
+    th[tid].fst = static_cast<float>(st);
+    th[tid].f = static_cast<float>(ct * dtheta * dphi * st);
+    th[tid].wy = ty.w;
+    th[tid].y0 = ty.i0;
+    th[tid].y1 = ty.i1;
+  }
+  __syncthreads();
   if (active) {
     const Taps tz = axis_taps(s_r_texel(J, r), J.nr);
     const Taps tx = axis_taps(s_mus_texel(J, mu_s), nmus);
     const float kR = static_cast<float>(3.0 / (16.0 * kPi));
     const double gd = J.g;
     const float kM = static_cast<float>(3.0 / (8.0 * kPi) * (1.0 - gd * gd) / (2.0 + gd * gd));
-    for (int e = lane; e < kTheta * nnu; e += 64) {
-      const int jt = e / nnu, n = e % nnu;
-      const double theta = (jt + 0.5) * dtheta;
-      const double ct = cos(theta);
-      const Taps ty = axis_taps(s_mu_texel(J, r, ct, false), nmu);
-      const float f = static_cast<float>(ct * dtheta * dphi * sin(theta));
-      const int zs[2] = {tz.i0, tz.i1}, ys[2] = {ty.i0, ty.i1}, xs[2] = {tx.i0, tx.i1};
-      const float wz[2] = {1.f - tz.w, tz.w}, wy[2] = {1.f - ty.w, ty.w},
+    const int entries = kTheta * nnu;
+    for (int e = tid; e < (one ? 2 : 1) * entries; e += kIiBlock) {
+      const int which = e >= entries ? 1 : 0;
+      const int jt = (e - which * entries) / nnu, n = (e - which * entries) % nnu;
+      const float f = th[jt].f;
+      const int zs[2] = {tz.i0, tz.i1}, ys[2] = {th[jt].y0, th[jt].y1}, xs[2] = {tx.i0, tx.i1};
+      const float wz[2] = {1.f - tz.w, tz.w}, wy[2] = {1.f - th[jt].wy, th[jt].wy},
                   wx[2] = {1.f - tx.w, tx.w};
       const int n1 = n + 1 < nnu ? n + 1 : n;
-      for (int which = 0; which < (one ? 2 : 1); ++which) {
-        const float4* src = which == 0 ? J.dR : J.dM;
-        const float fk = f * (one ? (which == 0 ? kR : kM) : 1.0f);
-        float3 v = make_float3(0.f, 0.f, 0.f), vn = make_float3(0.f, 0.f, 0.f);
-        for (int a = 0; a < 2; ++a)
-          for (int b = 0; b < 2; ++b)
-            for (int c = 0; c < 2; ++c) {
-              const float w = wz[a] * wy[b] * wx[c];
-              const int64_t base = (static_cast<int64_t>(zs[a]) * nmu + ys[b]) * W + xs[c];
-              const float4 p = gload(src, base + n * nmus), q = gload(src, base + n1 * nmus);
-              v.x += w * p.x;
-              v.y += w * p.y;
-              v.z += w * p.z;
-              vn.x += w * q.x;
-              vn.y += w * q.y;
-              vn.z += w * q.z;
-            }
-        v.x *= fk;
-        v.y *= fk;
-        v.z *= fk;
-        vn.x *= fk;
-        vn.y *= fk;
-        vn.z *= fk;
-        float4* tab = (which == 0 ? tab_a : tab_b) + jt * stride;
-        put_entry(tab, n + 1, v, vn);
-        if (n == 0) put_entry(tab, 0, v, v);
-      }
+      const float4* src = which == 0 ? J.dR : J.dM;
+      const float fk = f * (one ? (which == 0 ? kR : kM) : 1.0f);
+      float3 v = make_float3(0.f, 0.f, 0.f), vn = make_float3(0.f, 0.f, 0.f);
+      for (int a = 0; a < 2; ++a)
+        for (int b = 0; b < 2; ++b)
+          for (int c = 0; c < 2; ++c) {
+            const float w = wz[a] * wy[b] * wx[c];
+            const int64_t base = (static_cast<int64_t>(zs[a]) * nmu + ys[b]) * W + xs[c];
+            const float4 p = gload(src, base + n * nmus), q = gload(src, base + n1 * nmus);
+            v.x += w * p.x;
+            v.y += w * p.y;
+            v.z += w * p.z;
+            vn.x += w * q.x;
+            vn.y += w * q.y;
+            vn.z += w * q.z;
+          }
+      v.x *= fk;
+      v.y *= fk;
+      v.z *= fk;
+      vn.x *= fk;
+      vn.y *= fk;
+      vn.z *= fk;
+      float4* tab = (which == 0 ? tab_a : tab_b) + jt * stride;
+      put_entry(tab, n + 1, v, vn);
+      if (n == 0) put_entry(tab, 0, v, v);
     }
   }
   __syncthreads();
-  if (!active) return;
+  if (!active || tid >= 64) return;
   const double phi = (lane + 0.5) * dphi;
   const float wsx = static_cast<float>(sqrt(1.0 - mu_s * mu_s) * cos(phi));
   const float fmus = static_cast<float>(mu_s);
@@ -1046,8 +1065,7 @@ __global__ __launch_bounds__(64) void k_indirect_irradiance(
   const float mg2 = static_cast<float>(-2.0 * J.g);
   float a0 = 0.f, a1 = 0.f, a2 = 0.f;
   for (int jt = 0; jt < kTheta; ++jt) {
-    const double theta = (jt + 0.5) * dtheta;
-    const float ct = static_cast<float>(cos(theta)), st = static_cast<float>(sin(theta));
+    const float ct = th[jt].fct, st = th[jt].fst;
     const float nu = fmaf(st, wsx, ct * fmus);  // omega . omega_s
     float3 v = table_lerp(tab_a + jt * stride, fmaf(nu, hn, hn1));
     if (one) {
@@ -1886,7 +1904,7 @@ hipError_t launch_indirect_irradiance(const PassLaunch& p, int order,
                                       hipStream_t s) {
   const size_t lds =
       sizeof(float4) * static_cast<size_t>((order == 1 ? 4 : 2) * kTheta * (p.max_nnu + 1));
-  hipLaunchKernelGGL(k_indirect_irradiance, dim3(p.total_blocks), dim3(64), lds, s,
+  hipLaunchKernelGGL(k_indirect_irradiance, dim3(p.total_blocks), dim3(kIiBlock), lds, s,
                      p.jobs, p.first_block, p.njobs, order);
   return hipGetLastError();
 }
