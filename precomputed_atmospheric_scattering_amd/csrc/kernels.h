@@ -108,51 +108,79 @@ ATMO_HD int sd_split(const Job& j) {
 }
 
 // Single scattering: blocks of 'block' texels of a packed row, for 'nit'
-// iterations of a model, ss_staged of them with the blended transmittance rows
-// of a sample in LDS (TW up to 4096: 98 KB at most for one). The figures are
-// at k_single_scattering.
+// iterations of a model. Where 'staged', the block blends the transmittance
+// rows of each sample in LDS for ss_rows of them; otherwise every texel gathers
+// its four transmittance texels.
+//
+// A staged block blends all TW columns for each sample, however few texels it
+// has, and has a barrier per sample. It is worth that where the texels are at
+// least a quarter of the columns, the waves of a block are mostly full, and two
+// blocks per CU hide the barriers. Measured on MI355X (ms; wl: wavelengths),
+// gathered | staged:
+//   row of 256, TW 256, 3 wl: 4096 rows .147 | .131, 256 rows .024 | .031
+//   row of 192, TW 256, 3 wl: 1344 rows .054 | .053; 128: 2048 rows .052 | .066
+//   row of 512, 2048 rows, 3 wl: TW 2048 .305 | .252, TW 4096 .357 | .69
+//   row of 65, 16128 rows, TW 4096: .34 | 9.0 (3 wl), 1.8 | 50 (15 wl)
+// Iterations share a block that gathers where three blocks per CU are left and
+// the lines that the block reads per sample, in each iteration 2 rows of at most
+// one line per texel, leave room in the 32 KB L1. Alone | shared: row of 65, 4032
+// rows, TW 256, 15 wl .48 | .365; row of 96, 10880 rows, TW 1024, 6 wl .59 | .85;
+// row of 32, TW 256, 15 wl: 2048 rows .126 | .117, 512 rows .046 | .069.
 constexpr int kSsIters = 5;
 constexpr int kSsRowBytes = 64 << 10;  // at most, if iterations share a block
-constexpr int kSsGroupBlocks = 512;
-constexpr ATMO_HD int ss_staged(int nit, int block) {
-  return block < kBlock ? 0 : (nit < 3 ? 1 : 2);
-}
+constexpr int kSsStagedWidth = 192;    // shortest row
+constexpr int kSsColumns = 4;          // at most, blended per texel
+constexpr int kSsStagedBlocks = 512;
+constexpr int kSsGatherBlocks = 768;
+constexpr int kSsGatherBytes = 24 << 10;
+constexpr ATMO_HD int ss_rows(int nit, bool staged) { return !staged ? 0 : (nit < 3 ? 1 : 2); }
 template <bool kF64>
 constexpr int kSsBuffers = kF64 ? 1 : 2;
-ATMO_HD size_t ss_row_bytes(const Job& j, int nit, int block) {
-  const size_t texels = static_cast<size_t>(ss_staged(nit, block)) * j.tw * 3;
+ATMO_HD size_t ss_row_bytes(const Job& j, int nit, bool staged) {
+  const size_t texels = static_cast<size_t>(ss_rows(nit, staged)) * j.tw * 3;
   return texels * (j.acc64 ? kSsBuffers<true> * sizeof(double)
                            : kSsBuffers<false> * sizeof(float));
 }
 struct SsTiling {
   int block;
+  bool staged;
   int nit;  // 0: the job is served by the blocks of an earlier iteration
   bool fixed;  // FP32 job of fixed_sums: k_single_scattering_fixed instead
   ATMO_HD explicit SsTiling(const Job& j) {
     const int w = j.nnu * j.nmus, most = j.niter < kSsIters ? j.niter : kSsIters;
-    block = w > kBlock ? 2 * kBlock : (w > 64 ? kBlock : 64);
-    const int64_t blocks = static_cast<int64_t>(j.nr) * j.nmu * ((w + block - 1) / block);
-    nit = 1;
+    const int wide = w > kBlock ? 2 * kBlock : kBlock;
     fixed = fixed_sums(j) && !j.acc64;
-    // Iterations share a block once that leaves two blocks per CU.
-    if (most > 1 && ss_row_bytes(j, most, block) <= kSsRowBytes && blocks >= kSsGroupBlocks) {
+    staged = w >= kSsStagedWidth && j.tw <= kSsColumns * (w < wide ? w : wide) &&
+             blocks(j, wide) >= kSsStagedBlocks &&
+             (most == 1 || ss_row_bytes(j, most, true) <= kSsRowBytes);
+    block = staged ? wide : (w > 64 ? kBlock : 64);
+    const int lines = (j.tw + 7) / 8 < w ? (j.tw + 7) / 8 : w;  // 8 texels each
+    const bool share = staged || (blocks(j, block) >= kSsGatherBlocks &&
+                                  most * 2 * lines * 128 <= kSsGatherBytes);
+    nit = 1;
+    if (most > 1 && share) {
       const int left = j.niter - j.it;
       nit = j.it % kSsIters != 0 ? 0 : (left < kSsIters ? left : kSsIters);
     }
   }
+  static ATMO_HD int64_t blocks(const Job& j, int block) {
+    return static_cast<int64_t>(j.nr) * j.nmu * ((j.nnu * j.nmus + block - 1) / block);
+  }
 };
 // PassLaunch::ss_kinds.
-constexpr int ss_kind(bool f64, int nit, int block) {
-  return 1 << ((f64 ? nit : 0) + (block > kBlock ? 2 : (block == kBlock ? 1 : 0)) * (kSsIters + 1));
+constexpr int ss_kind(bool f64, int nit, int block, bool staged) {
+  return 1 << ((f64 ? nit : 0) +
+               (block > kBlock ? 3 : staged ? 2 : block == kBlock ? 1 : 0) * (kSsIters + 1));
 }
-constexpr int kSsFixed = 1 << (3 * (kSsIters + 1));
+constexpr int kSsFixed = 1 << (4 * (kSsIters + 1));
 ATMO_HD int ss_kind(const Job& j) {
   const SsTiling t(j);
-  return t.nit == 0 ? 0 : t.fixed ? kSsFixed : ss_kind(j.acc64 != 0, t.nit, t.block);
+  return t.nit == 0 ? 0
+                    : t.fixed ? kSsFixed : ss_kind(j.acc64 != 0, t.nit, t.block, t.staged);
 }
 inline size_t ss_lds(const Job& j) {
   const SsTiling t(j);
-  return ss_row_bytes(j, t.nit, t.block);
+  return ss_row_bytes(j, t.nit, t.staged);
 }
 
 // Scattering density of orders >= 3 (density_arcs.h): a block of 8 waves

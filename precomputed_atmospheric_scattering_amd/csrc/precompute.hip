@@ -270,26 +270,26 @@ __device__ __forceinline__ void ss_store(const Job& J, int64_t t_idx, double dx,
 // iterations of a model: where along the view ray the sun is seen, and at
 // which transmittance texel, does not depend on the wavelength. The two
 // transmittance rows of a sample's radius are the same for all texels of the
-// packed row: for ss_staged of the iterations the block blends them, times the
-// view transmittance, into LDS, and a texel interpolates between two
-// neighbours there; for the others it gathers its four texels from memory
-// (16 bytes a lane, 16 L1 cycles each). With all of them gathered, and the
-// geometry found for each iteration, the pass issued vector instructions in 99%
-// of the cycles at the reference sizes with 79% of the L1's; with all staged
-// the LDS (FP64 rows, read at random) is what limits it. On MI355X, ms per Init
-// of one iteration per block all gathered | 5 iterations with 5, 4, 3, 2, 1, 0
-// staged:
+// packed row. With kStage the block blends them, for ss_rows of the iterations,
+// times the view transmittance, into LDS, and a texel interpolates between two
+// neighbours there; for the other iterations, and without kStage for all of
+// them, it gathers its four texels from memory (16 bytes a lane, 16 L1 cycles
+// each). With all of them gathered, and the geometry found for each iteration,
+// the pass issued vector instructions in 99% of the cycles at the reference
+// sizes with 79% of the L1's; with all staged the LDS (FP64 rows, read at
+// random) is what limits it. On MI355X, ms per Init of one iteration per block
+// all gathered | 5 iterations with 5, 4, 3, 2, 1, 0 staged:
 //   1.05M texels, 15 wavelengths   .80 | .77  .69  .65  .62  .68  .83
 //   16.8M, 15                      16.4 | 14.5 13.6 12.5 11.5 12.4 26
 // and of 3 iterations with 2, 1 staged .195, .207 (.39M texels; before .22). One
 // FP32 iteration, gathered | staged: .153 | .130 at 1.05M texels, 2.8 | 1.8 at
-// 16.8M. Rows of at most 64 texels are gathered by single waves: staged, 32
-// texels wide rows took .025 ms against .021 at 8192 texels.
+// 16.8M. Rows of at most 64 texels are gathered by single waves. Which blocks
+// stage, and which iterations share one: SsTiling.
 // kF64: the kernel serves the jobs with FP64 accumulators (illuminance
 // mode) and computes the sun-side lookups and the sums in FP64; otherwise it
 // serves the others. The instances are launched over the same blocks when a
 // launch holds several kinds; each returns at once on the others' jobs.
-template <bool kF64, int kNit, int kB>
+template <bool kF64, int kNit, int kB, bool kStage>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4))) void
 k_single_scattering(
     const Job* __restrict__ jobs, const int* __restrict__ first_block, int njobs) {
@@ -302,7 +302,9 @@ k_single_scattering(
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
   const SsTiling tl(J);
-  if ((J.acc64 != 0) != kF64 || tl.fixed || tl.nit != kNit || tl.block != kB) return;
+  if ((J.acc64 != 0) != kF64 || tl.fixed || tl.nit != kNit || tl.block != kB ||
+      tl.staged != kStage)
+    return;
   const int W = J.nnu * J.nmus;
   const int lb = blockIdx.x - first_block[ji];
   const int tiles = (W + kB - 1) / kB;
@@ -332,7 +334,7 @@ k_single_scattering(
   const float4* __restrict__ T[kNit];
 #pragma unroll
   for (int k = 0; k < kNit; ++k) T[k] = (&J)[k].T;
-  constexpr int kStaged = ss_staged(kNit, kB);
+  constexpr int kStaged = ss_rows(kNit, kStage);
   constexpr bool kTwo = kSsBuffers<kF64> == 2;
   float4 a[kStaged + 1], b[kStaged + 1];
   auto fetch = [&](int s, int c) {
@@ -1825,21 +1827,21 @@ hipError_t launch_direct_irradiance(const PassLaunch& p, hipStream_t s) {
                      p.jobs, p.first_block, p.njobs);
   return hipGetLastError();
 }
-template <bool kF64, int kNit, int kB>
+template <bool kF64, int kNit, int kB, bool kStage>
 void launch_ss(const PassLaunch& p, hipStream_t s) {
-  if (p.ss_kinds & ss_kind(kF64, kNit, kB))
-    hipLaunchKernelGGL((k_single_scattering<kF64, kNit, kB>), dim3(p.total_blocks), dim3(kB),
-                       p.ss_lds, s, p.jobs, p.first_block, p.njobs);
+  if (p.ss_kinds & ss_kind(kF64, kNit, kB, kStage))
+    hipLaunchKernelGGL((k_single_scattering<kF64, kNit, kB, kStage>), dim3(p.total_blocks),
+                       dim3(kB), kStage ? p.ss_lds : 0, s, p.jobs, p.first_block, p.njobs);
 }
-template <int kB>
+template <int kB, bool kStage>
 void launch_ss_block(const PassLaunch& p, hipStream_t s) {
   static_assert(kSsIters == 5, "one launch per group size");
-  launch_ss<false, 1, kB>(p, s);
-  launch_ss<true, 1, kB>(p, s);
-  launch_ss<true, 2, kB>(p, s);
-  launch_ss<true, 3, kB>(p, s);
-  launch_ss<true, 4, kB>(p, s);
-  launch_ss<true, 5, kB>(p, s);
+  launch_ss<false, 1, kB, kStage>(p, s);
+  launch_ss<true, 1, kB, kStage>(p, s);
+  launch_ss<true, 2, kB, kStage>(p, s);
+  launch_ss<true, 3, kB, kStage>(p, s);
+  launch_ss<true, 4, kB, kStage>(p, s);
+  launch_ss<true, 5, kB, kStage>(p, s);
 }
 template <int kTpt>
 void launch_ss_fixed(const PassLaunch& p, hipStream_t s) {
@@ -1849,9 +1851,10 @@ void launch_ss_fixed(const PassLaunch& p, hipStream_t s) {
 }
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s) {
   // One instance per kind of job (SsTiling); each skips the others.
-  launch_ss_block<64>(p, s);
-  launch_ss_block<kBlock>(p, s);
-  launch_ss_block<2 * kBlock>(p, s);
+  launch_ss_block<64, false>(p, s);
+  launch_ss_block<kBlock, false>(p, s);
+  launch_ss_block<kBlock, true>(p, s);
+  launch_ss_block<2 * kBlock, true>(p, s);
   if (p.ss_kinds & kSsFixed) {
     launch_ss_fixed<1>(p, s);
     launch_ss_fixed<2>(p, s);

@@ -1,0 +1,72 @@
+"""The launch rules of csrc/kernels.h (which kernel a job takes), compiled for
+the host: no GPU needed."""
+import itertools
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """f(jobs) -> per job (block, staged, nit, fixed, lds, fixed_sums, sd_split)."""
+    exe = str(tmp_path_factory.mktemp("rules") / "host_rules")
+    cxx = shutil.which("amdclang++") or "/opt/rocm/bin/amdclang++"
+    r = subprocess.run([cxx, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                        os.path.join(HERE, "cpp", "host_rules.cc"), "-o", exe],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+
+    def f(jobs):
+        text = "\n".join(" ".join(str(int(v)) for v in j) for j in jobs)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=60)
+        rows = [tuple(map(int, l.split())) for l in out.stdout.splitlines()]
+        assert out.returncode == 0 and len(rows) == len(jobs)
+        return rows
+    return f
+
+
+def job(tw=256, nr=32, nmu=128, nmus=32, nnu=8, niter=1, it=0, half=0, acc64=None):
+    return (tw, 64, nr, nmu, nmus, nnu, 64, niter, it, half,
+            niter > 1 if acc64 is None else acc64)
+
+
+ROWS = [(2, 2), (8, 4), (13, 5), (16, 4), (16, 6), (32, 4), (32, 6), (32, 8), (27, 11), (64, 8),
+        (64, 16), (512, 32), (4096, 32)]
+JOBS = [job(tw, nr, nmu, nmus, nnu, niter)
+        for tw, (nr, nmu), (nmus, nnu), niter in itertools.product(
+            (2, 64, 256, 512, 1024, 2048, 4096), ((2, 4), (8, 32), (32, 128), (64, 256)), ROWS,
+            (1, 2, 5, 7))]
+
+
+def test_staged_blocks_blend_no_more_than_they_save(rules):
+    # A staged block blends TW columns per sample and iteration for its texels.
+    staged = 0
+    for (tw, _, nr, nmu, nmus, nnu, _, niter, _, _, _), r in zip(JOBS, rules(JOBS)):
+        block, stage, nit, _, lds = r[:5]
+        w = nmus * nnu
+        if stage:
+            staged += 1
+            assert tw <= 4 * min(w, block) and w >= 192 and lds <= 64 << 10
+            assert nr * nmu * -(-w // block) >= 512
+        else:
+            assert lds == 0 and block <= 256
+        assert block >= 64 and nit in (1, niter if niter < 5 else 5)
+    assert 0 < staged < len(JOBS)
+
+
+def test_iterations_are_served_once(rules):
+    # The blocks of an iteration serve the nit - 1 that follow it.
+    for tw, nmus in itertools.product((64, 1024, 4096), (4, 32)):
+        for niter in range(1, 12):
+            rs = rules([job(tw, nmus=nmus, niter=niter, it=i) for i in range(niter)])
+            i = 0
+            while i < niter:
+                nit = rs[i][2]
+                assert 1 <= nit <= 5 and i + nit <= niter
+                assert all(rs[k][2] == 0 for k in range(i + 1, i + nit))
+                assert all(rs[k][:2] == rs[i][:2] for k in range(i, i + nit))
+                i += nit
