@@ -311,11 +311,12 @@ hipError_t launch_to_half(const PassLaunch& p, hipStream_t s);
 hipError_t launch_interleave(const PassLaunch& p, hipStream_t s);
 
 // Lookups (one ray / point per thread). 'job' is a device pointer, 'combined'
-// its Job::combined. With
+// its Job::combined, 'copy' whether it has a lookup copy (if that changes before a
+// captured launch runs, the kernels read S and SM themselves). With
 // 'luminance' the results are scaled by the job's radiance-to-luminance
 // factors (the Luminance API of atmosphere/model.cc:252-281).
-hipError_t launch_sky_radiance(const Job* job, bool combined, int64_t n, const float* camera,
-                               const float* view_ray,
+hipError_t launch_sky_radiance(const Job* job, bool combined, bool copy, int64_t n,
+                               const float* camera, const float* view_ray,
                                const float* shadow_length,
                                const float* sun_direction, float* radiance,
                                float* transmittance, int luminance, hipStream_t s);

@@ -143,10 +143,10 @@ __device__ __forceinline__ void lookup_lines(const Job& J, const SCoords& c, uin
 }
 
 // functions.glsl:1658-1690. kF32: FP32 tap weights and sums (lookups whose
-// result is not a difference of two lookups); otherwise FP64. kLines: S and SM
-// are separate; then all lanes of the wave call it, with the wave's kStageParts
-// parts of LDS.
-template <bool kF32, bool kLines>
+// result is not a difference of two lookups); otherwise FP64. kSeparate: S and
+// SM are separate. kLines: they may have a lookup copy; then all lanes of the wave
+// call it, with the wave's kStageParts parts of LDS.
+template <bool kF32, bool kSeparate, bool kLines>
 __device__ D4 combined_scattering(const Job& J, double r, double mu, double mu_s,
                                   double nu, bool ground, uint4* stage, D4* single_mie) {
   using Real = typename std::conditional<kF32, float, double>::type;
@@ -170,16 +170,16 @@ __device__ D4 combined_scattering(const Job& J, double r, double mu, double mu_s
     const F16Texels st{J.S16, make_float4(1.0f / sc[0], 1.0f / sc[1], 1.0f / sc[2],
                                           1.0f / sc[3])};
     s = lookup(st);
-    if (kLines) {
+    if (kSeparate) {
       const F16Texels mt{J.SM16, make_float4(1.0f / sc[4], 1.0f / sc[5], 1.0f / sc[6],
                                              0.0f)};
       *single_mie = rgb(lookup(mt));
     }
   } else {
     s = lookup(F32Texels{J.S});
-    if (kLines) *single_mie = rgb(lookup(F32Texels{J.SM}));
+    if (kSeparate) *single_mie = rgb(lookup(F32Texels{J.SM}));
   }
-  if (!kLines) *single_mie = extrapolated_mie(J, s);
+  if (!kSeparate) *single_mie = extrapolated_mie(J, s);
   return s;
 }
 
@@ -195,11 +195,11 @@ __device__ __forceinline__ D4 shade(const Job& J, D4 scat, D4 mie, double nu,
   return l;
 }
 
-// kLines: for models with separate S and SM (combined_scattering). Three waves
-// per SIMD take 168 VGPRs with lines (175 unbounded, 8% slower); without, the
-// loads in flight of fewer waves are worth more (FP16, scattered: 121 us for
-// 2.07M rays with 2, 131 with 3).
-template <bool kLines>
+// kSeparate, kLines: as in combined_scattering. Three waves per SIMD take 168
+// VGPRs with lines (175 unbounded, 8% slower); without, the loads in flight of
+// fewer waves are worth more (2.07M scattered rays with 2 waves, and 3: combined FP16 121
+// us, 131; separate without a copy 193, 241 FP16, 286, 313 FP32).
+template <bool kSeparate, bool kLines>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kLines ? 3 : 2))) void
 k_sky_radiance(
     const Job* __restrict__ job, int64_t n, const float* __restrict__ camera,
@@ -238,23 +238,38 @@ k_sky_radiance(
     r = J.rt;
     rmu = r;
   }
+  // With lines, a wave leaves together (most waves of a frame seen from space do:
+  // 2.07M pixels 40 us, 60 where each stays for the lookups).
+  if (kLines && __all(space)) {
+    if (ray >= n) return;
+    store3(transmittance_out, i, D4{1.0, 1.0, 1.0, 0.0});
+    store3(radiance, i, D4{0.0, 0.0, 0.0, 0.0});
+    return;
+  }
   const double mu = rmu / r;
   const double mu_s = dot3(cam, sd) / r;
   const double nu = dot3(v, sd);
   const bool ground = hits_ground(J, r, mu);
   const D4 zero{0.0, 0.0, 0.0, 0.0};
   const D4 t = ground ? zero : t_lookup_d(J, J.T, r, mu);
-  double r_p = r, mu_p = mu, mu_s_p = mu_s;
-  if (shadow != 0.0) {
-    // Light shafts (functions.glsl:1746-1766).
-    const double d = shadow;
-    r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
-    mu_p = (r * mu + d) / r_p;
-    mu_s_p = (r * mu_s + d * nu) / r_p;
+  D4 mie, scat;
+  if (kSeparate && !kLines && shadow == 0.0) {
+    // (Without a copy, a lookup of its own for these rays: 300k scattered rays with
+    // light shafts 65 us with one for both, high-resolution LUTs, 56 with two.)
+    scat = combined_scattering<true, kSeparate, kLines>(J, r, mu, mu_s, nu, ground, stage, &mie);
+  } else {
+    double r_p = r, mu_p = mu, mu_s_p = mu_s;
+    if (shadow != 0.0) {
+      // Light shafts (functions.glsl:1746-1766).
+      const double d = shadow;
+      r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
+      mu_p = (r * mu + d) / r_p;
+      mu_s_p = (r * mu_s + d * nu) / r_p;
+    }
+    scat = combined_scattering<true, kSeparate, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage,
+                                                        &mie);
   }
-  D4 mie;
-  D4 scat = rgb(combined_scattering<true, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage,
-                                                  &mie));
+  scat = rgb(scat);
   if (ray >= n) return;
   if (shadow != 0.0) {
     const D4 st = transmittance_d(J, J.T, r, mu, shadow, ground);
@@ -306,7 +321,8 @@ k_sky_radiance_to_point(
   const D4 here = t_lookup_d(J, J.T, r, ground ? -mu : mu);
   const D4 t = transmittance_from_d(J, J.T, here, r, mu, d, ground);
   D4 mie;
-  D4 scat = rgb(combined_scattering<false, kLines>(J, r, mu, mu_s, nu, ground, stage, &mie));
+  D4 scat =
+      rgb(combined_scattering<false, kLines, kLines>(J, r, mu, mu_s, nu, ground, stage, &mie));
   // functions.glsl:1831-1840
   d = d - shadow > 0.0 ? d - shadow : 0.0;
   const double r_p = clamp_radius(J, sqrt(d * d + 2.0 * r * mu * d + r * r));
@@ -314,7 +330,8 @@ k_sky_radiance_to_point(
   const double mu_s_p = (r * mu_s + d * nu) / r_p;
   D4 mie_p;
   const D4 scat_p =
-      rgb(combined_scattering<false, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage, &mie_p));
+      rgb(combined_scattering<false, kLines, kLines>(J, r_p, mu_p, mu_s_p, nu, ground, stage,
+                                                     &mie_p));
   if (ray >= n) return;
   D4 st = t;
   if (shadow > 0.0) st = transmittance_from_d(J, J.T, here, r, mu, d, ground);
@@ -411,13 +428,14 @@ inline unsigned grid_for(int64_t n) {
 
 }  // namespace
 
-hipError_t launch_sky_radiance(const Job* job, bool combined, int64_t n, const float* camera,
-                               const float* view_ray,
+hipError_t launch_sky_radiance(const Job* job, bool combined, bool copy, int64_t n,
+                               const float* camera, const float* view_ray,
                                const float* shadow_length,
                                const float* sun_direction, float* radiance,
                                float* transmittance, int luminance, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  const auto kernel = combined ? k_sky_radiance<false> : k_sky_radiance<true>;
+  const auto kernel = combined ? k_sky_radiance<false, false>
+                      : copy ? k_sky_radiance<true, true> : k_sky_radiance<true, false>;
   hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, job, n, camera, view_ray,
                      shadow_length, sun_direction, radiance, transmittance, luminance);
   return hipGetLastError();

@@ -1156,7 +1156,8 @@ static atmo_status sky(const atmo_model* m, int64_t n, const float* camera,
   if (n > 0 && (!camera || !view_ray || !shadow_length || !sun_direction || !radiance ||
                 !transmittance))
     return fail(ATMO_ERROR_INVALID_ARGUMENT, "NULL array");
-  return check_launch(atmo::launch_sky_radiance(query_job(m), m->spec.combined, n, camera,
+  return check_launch(atmo::launch_sky_radiance(query_job(m), m->spec.combined,
+                                                m->Q != nullptr, n, camera,
                                                 view_ray, shadow_length, sun_direction,
                                                 radiance, transmittance, luminance,
                                                 static_cast<hipStream_t>(stream)),
