@@ -107,6 +107,9 @@ struct Job {
   // model's rows sorted by the impact parameter of their view ray).
   int ms_row_order;
   const int* ms_rows;
+  // ms_pairs and ms_spread of kernels.h (their divisions took each block a
+  // microsecond).
+  int ms_paired, ms_spread_out;
   // LUT sizes.
   int tw, th;
   int nr, nmu, nmus, nnu;

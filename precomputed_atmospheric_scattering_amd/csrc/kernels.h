@@ -23,7 +23,7 @@ struct PassLaunch {
   int kinds;    // kJobsF32 | kJobsAcc64: which kinds of jobs the launch holds
   int tile;     // tile shape of the jobs (scattering density, multiple
                 // scattering): every job of a launch has the same one
-  int dj_kinds;  // kDjF32 | kDjRgb21: the delta J formats of the jobs
+  int dj_kinds;  // dj_kind of the jobs, or-ed
   int ss_kinds;    // ss_kind of the jobs, or-ed
   size_t ss_lds;   // largest ss_lds of the jobs
   int sd_kinds;    // 1 << sd_split of the jobs, or-ed
@@ -33,6 +33,7 @@ struct PassLaunch {
 
 constexpr int kDjF32 = 1;    // delta J as RGB float (FP32-storage jobs)
 constexpr int kDjRgb21 = 2;  // delta J as 3 x 21-bit floats (FP16-storage jobs)
+constexpr int kDjPairs = 4;  // the same, read two texels at a time (ms_pairs)
 
 constexpr int kJobsF32 = 1;    // jobs accumulating S and SM in FP32
 constexpr int kJobsAcc64 = 2;  // illuminance-mode jobs with FP64 accumulators
@@ -241,6 +242,42 @@ ATMO_HD int ms_rows_per_block(int w, int capacity) {
 ATMO_HD int ms_tile_rows(int w, int tpt, int block) {
   const int r = ms_rows_per_block(w, tpt * block), m = block / ((w + tpt - 1) / tpt);
   return r < m ? r : m;
+}
+// Whether the threads of an FP16 job load two neighbouring texels of delta J. With
+// one texel per thread, half of a block's waves then load, which a launch of few
+// blocks waits for. Measured on MI355X, us, a texel at a time | two (15 wavelengths
+// unless given):
+//   rows of 256: 1024 blocks (3 wl) 48 | 48, 5120 171 | 168, 20480 645 | 620;
+//     64 (3 wl) 31 | 35
+//   rows of 64: 256 blocks (3 wl) 31 | 35, 1280 64 | 68, 5120 179 | 183
+//   rows of 32: 2560 blocks 146 | 126, 640 52 | 51, 128 (3 wl) 29 | 32
+//   rows of 96, in 192 of the 256 threads: 2048 blocks (3 wl) 65 | 69, 10240 279 | 290
+// With two texels per thread every wave loads either way: rows of 1024, 64 rows
+// (3 wl) 61 | 49.
+constexpr int kMsPairBlocks = 2048;
+constexpr int kMsPairShort = 32, kMsPairLong = 128;  // not the rows between
+ATMO_HD bool ms_pairs(const Job& j) {
+  if (j.half_luts == 0) return false;
+  const MsTile t = kMsTile[j.ms_tile];
+  if (t.tpt > 1) return true;
+  const int w = j.nnu * j.nmus, rpb = ms_tile_rows(w, t.tpt, t.block);
+  if (rpb <= 0 || (w > kMsPairShort && w < kMsPairLong)) return false;
+  const int64_t rows = static_cast<int64_t>(j.nr) * j.nmu;
+  return (rows + rpb - 1) / rpb * j.niter >= kMsPairBlocks;
+}
+// Whether the two texels of a thread are a block's width apart, so that all waves of
+// a block with one row have texels, and not half a row, which leaves some waves idle
+// and the others full. Better where a CU has one block: rows of 640 texels, FP32, us,
+// half a row | a block apart: 64 blocks 53 | 47, 256 56 | 50, 320 62 | 68, 1024 119 |
+// 125.
+constexpr int kMsSpreadBlocks = 256;
+ATMO_HD bool ms_spread(const Job& j) {
+  const MsTile t = kMsTile[j.ms_tile];
+  return j.half_luts == 0 && t.tpt > 1 && ms_tile_rows(j.nnu * j.nmus, t.tpt, t.block) == 1 &&
+         static_cast<int64_t>(j.nr) * j.nmu * j.niter <= kMsSpreadBlocks;
+}
+ATMO_HD int dj_kind(const Job& j) {
+  return j.half_luts == 0 ? kDjF32 : (j.ms_paired ? kDjPairs : kDjRgb21);
 }
 // The smallest tile that holds a row of w texels.
 ATMO_HD int ms_default_tile(int w) {

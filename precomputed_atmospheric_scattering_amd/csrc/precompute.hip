@@ -1119,7 +1119,7 @@ __global__ __launch_bounds__(kIiBlock) void k_indirect_irradiance(
 // Each of the kB threads holds kTpt texels of one row, whose samples it reads
 // once; a block takes ms_tile_rows whole rows (several short rows, or one row
 // of up to kTpt * kB texels). FP16 models' threads load two neighbouring texels
-// at a time: at rows of 1024 texels and 15 wavelengths 75.5 ms per Init of 8
+// at a time, but for launches of few blocks (ms_pairs): at rows of 1024 texels and 15 wavelengths 75.5 ms per Init of 8
 // orders against 81.0 with a load per texel and the samples read for each (the
 // address units busy 45% of the time instead of 65%; then the LDS is, 81%); at
 // rows of 256, 1.90 ms against 1.97 (4 orders); FP32 rows of 1024 with 3
@@ -1190,12 +1190,16 @@ struct MsRowSample {
   float pad;
 };
 
-// A load of delta J at a byte offset: 12 bytes, or two 8-byte texels.
+// A load of delta J at a byte offset: a texel of 12 or 8 bytes, or two of 8.
 template <class T>
 __device__ __forceinline__ T ms_load(const char* __restrict__ D, uint32_t at);
 template <>
 __device__ __forceinline__ float3 ms_load<float3>(const char* __restrict__ D, uint32_t at) {
   return gload_at(reinterpret_cast<const float3*>(D), at);
+}
+template <>
+__device__ __forceinline__ uint2 ms_load<uint2>(const char* __restrict__ D, uint32_t at) {
+  return gload_at(reinterpret_cast<const uint2*>(D), at);
 }
 template <>
 __device__ __forceinline__ uint4 ms_load<uint4>(const char* __restrict__ D, uint32_t at) {
@@ -1211,7 +1215,7 @@ __device__ __forceinline__ uint4 ms_load<uint4>(const char* __restrict__ D, uint
 // One texel per thread (rows up to 256 texels): eight waves per SIMD (64
 // VGPRs, 32 bytes of spills) measured 2% faster than six at the reference
 // sizes; the two-texel shapes keep the compiler's allocation.
-template <int kTpt, bool kF16, int kB>
+template <int kTpt, bool kF16, int kB, bool kPairs>
 __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
     const Job* __restrict__ jobs, const int* __restrict__ first_block,
     int njobs, int max_rows) {
@@ -1225,6 +1229,7 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   const int ji = find_job(first_block, njobs, blockIdx.x);
   const Job& J = jobs[ji];
   if ((J.half_luts != 0) != kF16) return;
+  if (kF16 && (J.ms_paired != 0) != kPairs) return;
   const int lb = blockIdx.x - first_block[ji];
   const int nnu = J.nnu, nmus = J.nmus, nmu = J.nmu;
   const int W = nnu * nmus;
@@ -1281,7 +1286,8 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   // blended row (the slice's first texel).
   // The texels of a thread are in one row, x and x + tpr: its samples are read
   // once.
-  const int tpr = (W + kTpt - 1) / kTpt;  // threads per row
+  const int tpr =  // threads per row
+      kTpt > 1 && !kF16 && J.ms_spread_out && rpb == 1 ? kB : (W + kTpt - 1) / kTpt;
   const int slot = tid / tpr < rpb && row0 + tid / tpr < nrows ? tid / tpr : -1;
   int x_of[kTpt];  // or -1
   uint32_t c0_of[kTpt], c1_of[kTpt];
@@ -1323,23 +1329,22 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   __syncthreads();
 
   const MusMap mus_map(J);
-  // What a thread blends. FP32: its texels. FP16: two neighbours, with 16-byte
+  // What a thread blends: its texels, or (kPairs) two neighbours, with 16-byte
   // loads (a load of 64 lanes costs 16 cycles at 8, 12 or 16 bytes a lane);
-  // the last pair of an odd row overlaps the one before it. With one texel per
-  // thread, half of the waves blend.
-  constexpr int kLoads = kF16 ? 1 : kTpt;
-  using Load = typename std::conditional<kF16, uint4, float3>::type;
-  const int ppr = kF16 ? (W + 1) / 2 : tpr;  // threads that blend per row
-  const int from = kTpt == 1 && kF16
-                       ? (tid / ppr < rpb && row0 + tid / ppr < nrows ? tid / ppr : -1)
-                       : slot;
+  // the last pair of an odd row overlaps the one before it.
+  constexpr int kLoads = kPairs ? 1 : kTpt;
+  using Load = typename std::conditional<
+      kPairs, uint4, typename std::conditional<kF16, uint2, float3>::type>::type;
+  const int ppr = (W + 1) / 2;  // threads that blend per row, with kPairs
+  const int from =
+      kPairs ? (tid / ppr < rpb && row0 + tid / ppr < nrows ? tid / ppr : -1) : slot;
   const MsRowSample* const blend = smp[from < 0 ? 0 : from];
   const MsRowSample* const march = smp[slot < 0 ? 0 : slot];
-  const int pair = kF16 ? min(2 * (tid - tid / ppr * ppr), W - 2) : 0;
+  const int pair = kPairs ? min(2 * (tid - tid / ppr * ppr), W - 2) : 0;
   uint32_t x_bytes[kLoads], to[kLoads];  // in a source row; in a buffer
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) {
-    const int x = kF16 ? pair : (x_of[j] < 0 ? 0 : x_of[j]);
+    const int x = kPairs ? pair : (x_of[j] < 0 ? 0 : x_of[j]);
     x_bytes[j] = static_cast<uint32_t>(x) * static_cast<uint32_t>(kF16 ? 8 : 12);
     to[j] = static_cast<uint32_t>((from < 0 ? 0 : from) * W + x);
   }
@@ -1348,9 +1353,9 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
   // loads are in flight during the barrier and the gather of the current one.
   Load src[kLoads][4];
   auto fetch = [&](int i) {
-    // FP32: idle lanes load row slot 0's texel 0, in bounds, so that the loads
-    // need no branch.
-    if (kF16 && from < 0) return;
+    // A texel at a time: idle lanes load row slot 0's texel 0, in bounds, so that
+    // the loads need no branch.
+    if (kPairs && from < 0) return;
     const MsRowSample& S = blend[i];
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
@@ -1374,7 +1379,7 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
       };
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
-        if constexpr (kF16) {
+        if constexpr (kPairs) {
           auto half = [&](int k, int c) {
             return unpack_f21x3(c == 0 ? make_uint2(src[j][k].x, src[j][k].y)
                                        : make_uint2(src[j][k].z, src[j][k].w));
@@ -1382,7 +1387,11 @@ __global__ __launch_bounds__(kB, kTpt == 1 ? 8 : 1) void k_multiple_scattering(
           B[to[j]] = mix(half(0, 0), half(1, 0), half(2, 0), half(3, 0));
           B[to[j] + 1] = mix(half(0, 1), half(1, 1), half(2, 1), half(3, 1));
         } else if (x_of[j] >= 0) {
-          B[to[j]] = mix(src[j][0], src[j][1], src[j][2], src[j][3]);
+          if constexpr (kF16)
+            B[to[j]] = mix(unpack_f21x3(src[j][0]), unpack_f21x3(src[j][1]),
+                           unpack_f21x3(src[j][2]), unpack_f21x3(src[j][3]));
+          else
+            B[to[j]] = mix(src[j][0], src[j][1], src[j][2], src[j][3]);
         }
       }
     }
@@ -1941,12 +1950,14 @@ void launch_ms_tile(const PassLaunch& p, hipStream_t s) {
   const int rows = ms_rows_per_block(p.min_w, kTpt * kB);
   const size_t lds = sizeof(float3) * 2 * kB * kTpt +
                      sizeof(MsRowSample) * kMarch * static_cast<size_t>(rows);
-  if (p.dj_kinds & kDjF32)
-    hipLaunchKernelGGL((k_multiple_scattering<kTpt, false, kB>), dim3(p.total_blocks),
-                       dim3(kB), lds, s, p.jobs, p.first_block, p.njobs, rows);
-  if (p.dj_kinds & kDjRgb21)
-    hipLaunchKernelGGL((k_multiple_scattering<kTpt, true, kB>), dim3(p.total_blocks),
-                       dim3(kB), lds, s, p.jobs, p.first_block, p.njobs, rows);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(p.total_blocks), dim3(kB), lds, s, p.jobs, p.first_block,
+                       p.njobs, rows);
+  };
+  if (p.dj_kinds & kDjF32) launch(k_multiple_scattering<kTpt, false, kB, false>);
+  if (p.dj_kinds & kDjPairs) launch(k_multiple_scattering<kTpt, true, kB, true>);
+  if constexpr (kTpt == 1)
+    if (p.dj_kinds & kDjRgb21) launch(k_multiple_scattering<kTpt, true, kB, false>);
 }
 
 hipError_t launch_multiple_scattering(const PassLaunch& p, hipStream_t s) {

@@ -488,6 +488,8 @@ void fill_job_luts(atmo_model* m, atmo::Job* j, int k) {
   j->ms_tile = t.ms;
   j->ms_row_order = t.ms_row_order;
   j->ms_rows = m->d_ms_rows;
+  j->ms_paired = atmo::ms_pairs(*j) ? 1 : 0;
+  j->ms_spread_out = atmo::ms_spread(*j) ? 1 : 0;
 }
 
 // Rebuild the host job table (LUT pointers may have changed) and upload it.
@@ -541,8 +543,8 @@ atmo::PassLaunch model_launch(const atmo_model* m, int first_job, int njobs, Pas
   l.min_w = l.max_w;
   l.max_lds_w = l.max_w <= atmo::kMsMaxRow ? l.max_w : 0;
   l.kinds = accumulates_fp64(m->spec) ? atmo::kJobsAcc64 : atmo::kJobsF32;
-  l.dj_kinds = m->spec.half_precision ? atmo::kDjRgb21 : atmo::kDjF32;
   const atmo::Job& j = m->jobs[first_job];
+  l.dj_kinds = atmo::dj_kind(j);
   l.sd_kinds = 1 << atmo::sd_split(j);
   l.ss_kinds = l.arc_kinds = 0;
   l.ss_lds = 0;
@@ -1480,7 +1482,7 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
       if (j.nnu * j.nmus <= atmo::kMsMaxRow)
         l.max_lds_w = std::max(l.max_lds_w, j.nnu * j.nmus);
       l.kinds |= j.acc64 ? atmo::kJobsAcc64 : atmo::kJobsF32;
-      l.dj_kinds |= j.half_luts ? atmo::kDjRgb21 : atmo::kDjF32;
+      l.dj_kinds |= atmo::dj_kind(j);
       l.ss_kinds |= atmo::ss_kind(j);
       l.ss_lds = std::max(l.ss_lds, atmo::ss_lds(j));
       l.sd_kinds |= 1 << atmo::sd_split(j);

@@ -12,7 +12,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
-    """f(jobs) -> per job (block, staged, nit, fixed, lds, fixed_sums, sd_split)."""
+    """f(jobs) -> per job (block, staged, nit, fixed, lds, fixed_sums, sd_split,
+    ms_pairs, ms_spread)."""
     exe = str(tmp_path_factory.mktemp("rules") / "host_rules")
     cxx = shutil.which("amdclang++") or "/opt/rocm/bin/amdclang++"
     r = subprocess.run([cxx, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
@@ -70,3 +71,19 @@ def test_iterations_are_served_once(rules):
                 assert all(rs[k][2] == 0 for k in range(i + 1, i + nit))
                 assert all(rs[k][:2] == rs[i][:2] for k in range(i, i + nit))
                 i += nit
+
+
+def test_few_blocks_load_texel_by_texel(rules):
+    # Rows of 256 texels, one per block of one-texel threads; rows of 96 at any size.
+    assert [r[7] for r in rules([job(nr=8, nmu=32, half=1), job(nr=32, nmu=64, half=1),
+                                 job(nr=31, nmu=66, half=1), job(nr=16, nmu=26, niter=5, half=1),
+                                 job(nr=32, nmu=128), job(nr=2, nmu=4, nmus=64, half=1),
+                                 job(nr=64, nmu=256, nmus=16, nnu=6, niter=5, half=1)])] == [
+        0, 1, 0, 1, 0, 1, 0]
+    # FP32 rows of 640 alone in a block.
+    assert [r[8] for r in rules([job(nr=8, nmu=32, nmus=64, nnu=10),
+                                 job(nr=8, nmu=34, nmus=64, nnu=10),
+                                 job(nr=2, nmu=24, nmus=64, nnu=10, niter=5),
+                                 job(nr=2, nmu=26, nmus=64, nnu=10, niter=5),
+                                 job(nr=8, nmu=32, nmus=64, nnu=10, half=1), job(nr=2, nmu=4)])
+            ] == [1, 0, 1, 0, 0, 0]
