@@ -238,8 +238,9 @@ void atmo_batch_destroy(atmo_batch* batch);
  * passes are fragment-shader draws). The scattering density, where it is
  * summed direction by direction with a thread per output (order 2 of LUTs of
  * more than 1.25M texels times Precompute iterations; every order of
- * half-precision models of up to 2^22 texels), runs with sd_nu_per_thread nu
- * outputs per thread in blocks of sd_block_threads. The multiple-scattering
+ * half-precision models of up to 2^22 texels, and of models of 3 wavelengths
+ * with 20 or more NU and 1.9M texels), runs with sd_nu_per_thread nu outputs
+ * per thread in blocks of sd_block_threads. The multiple-scattering
  * pass runs with ms_texels_per_thread texels per thread in blocks of
  * ms_block_threads, its blocks walking the (r, mu) rows of the LUT r-major
  * (ms_row_order 0, the LUT's own order), mu-major (1) or in ray order (2: rows sorted by the

@@ -79,6 +79,21 @@ ATMO_HD bool fixed_sums(const Job& j) {
          static_cast<int64_t>(j.nr) * j.nmu * j.nmus * j.nnu <= kFixedTexels;
 }
 
+// Whether the density of the orders >= 3 is made of arc sums (density_arcs.h) or
+// direction by direction. The arcs' terms serve all iterations of a model, and are
+// 2 + 2/3 NU in number: with one iteration and many NU the directions are faster.
+// Measured on MI355X, ms per order, 3 wavelengths, directions | arcs:
+//   NU 16, 16.8M texels 2.9 | 2.8;  NU 20, 2.6M .55 | .54, 5.2M .99 | 1.07
+//   NU 24, 1.6M .42 | .40, 2.0M .42 | .48, 3.1M .60 | .73, 12.6M 2.24 | 2.88
+//   NU 32, 2.1M .45 | .49, 8.4M 1.66 | 1.89
+// With 6 wavelengths the arcs are 1.4 times as fast at the least.
+constexpr int kArcMaxNu = 20;
+constexpr int64_t kArcTexels = 1900000;
+ATMO_HD bool arc_sums(const Job& j) {
+  const int64_t n = static_cast<int64_t>(j.nr) * j.nmu * j.nmus * j.nnu;
+  return !fixed_sums(j) && !(j.niter == 1 && j.nnu >= kArcMaxNu && n >= kArcTexels);
+}
+
 // Grids too small to fill the GPU at 4 outputs per thread: several threads
 // share an output, each summing some of the zenith angles, whatever the tile
 // shape. A job takes the first of these whose 'texels' it does not exceed (of
@@ -324,7 +339,7 @@ hipError_t launch_transmittance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_direct_irradiance(const PassLaunch& p, hipStream_t s);
 hipError_t launch_single_scattering(const PassLaunch& p, hipStream_t s);
 // The scattering density direction by direction (order 2, and the orders >= 3
-// of the fixed_sums jobs), and that of an order >= 3 by arc sums. In the
+// of the jobs that are not arc_sums), and that of an order >= 3 by arc sums. In the
 // latter the jobs of a model's Precompute iterations follow each other in
 // p.jobs, and the blocks of the first of every kArcIters serve all of them.
 hipError_t launch_scattering_density(const PassLaunch& p, int order, hipStream_t s);

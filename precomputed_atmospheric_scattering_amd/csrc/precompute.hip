@@ -766,7 +766,7 @@ __device__ __forceinline__ void sd_theta(
 // kParts: threads that share an output, each summing kTheta / kParts of the
 // zenith angles (kSdSplit; 1 for the jobs that take none of it).
 // kTwo: order 2; otherwise an order >= 3 of the models that do not take the arc
-// sums (fixed_sums), never in parts.
+// sums (arc_sums), never in parts.
 template <int kChunk, int kB, int kParts, bool kTwo>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(5))) void
 k_scattering_density(

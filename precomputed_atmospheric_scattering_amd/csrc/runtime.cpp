@@ -630,7 +630,7 @@ atmo_status enqueue_precompute(atmo_model* m, unsigned orders, LaunchTimer& t) {
   for (unsigned order = 2; order <= orders; ++order) {
     const int o = static_cast<int>(order);
     ATMO_TRY(t.run(kSD, o, "scattering density", [&] {
-      return order == 2 || atmo::fixed_sums(m->jobs[0])
+      return order == 2 || !atmo::arc_sums(m->jobs[0])
                  ? atmo::launch_scattering_density(model_launch(m, 0, n, kSD), order, s)
                  : atmo::launch_density_arcs(model_launch(m, 0, n, kSA), s);
     }));
@@ -1532,7 +1532,7 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
       if (orders[mj.first] >= n) on.push_back(mj);
     std::vector<std::pair<int, int>> direct, arcs;
     for (const auto& mj : on)
-      (n == 2 || atmo::fixed_sums(models[mj.first]->jobs[0]) ? direct : arcs).push_back(mj);
+      (n == 2 || !atmo::arc_sums(models[mj.first]->jobs[0]) ? direct : arcs).push_back(mj);
     add_level(kSD, static_cast<int>(n), direct);
     add_level(kSA, static_cast<int>(n), arcs);
     add_level(kII, static_cast<int>(n) - 1, on);

@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
     """f(jobs) -> per job (block, staged, nit, fixed, lds, fixed_sums, sd_split,
-    ms_pairs, ms_spread)."""
+    ms_pairs, ms_spread, arc_sums)."""
     exe = str(tmp_path_factory.mktemp("rules") / "host_rules")
     cxx = shutil.which("amdclang++") or "/opt/rocm/bin/amdclang++"
     r = subprocess.run([cxx, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
@@ -87,3 +87,18 @@ def test_few_blocks_load_texel_by_texel(rules):
                                  job(nr=2, nmu=26, nmus=64, nnu=10, niter=5),
                                  job(nr=8, nmu=32, nmus=64, nnu=10, half=1), job(nr=2, nmu=4)])
             ] == [1, 0, 1, 0, 0, 0]
+
+
+def test_arc_sums(rules):
+    # 3 wavelengths: NU 20 and more from 1.9M texels on take the directions; so do
+    # FP16-storage models of up to 2^22 texels.
+    jobs = [job(nr=64, nmu=256, nmus=64, nnu=16), job(nr=32, nmu=128, nmus=32, nnu=19),
+            job(nr=32, nmu=128, nmus=32, nnu=20), job(nr=32, nmu=128, nmus=20, nnu=23),
+            job(nr=32, nmu=128, nmus=20, nnu=24), job(nr=32, nmu=128, nmus=20, nnu=32, niter=2),
+            job(nr=32, nmu=128, half=1), job(nr=64, nmu=128, nmus=64, nnu=8, half=1),
+            job(nr=64, nmu=128, nmus=64, nnu=9, half=1), job(nr=64, nmu=128, nmus=64, half=1,
+                                                             nnu=20)]
+    got = rules(jobs)
+    assert [r[9] for r in got] == [1, 1, 0, 1, 0, 1, 0, 0, 1, 0]
+    # What is summed by directions at the orders >= 3 has a thread per output.
+    assert all(r[6] == 3 for r in got if not r[9])
