@@ -381,28 +381,43 @@ struct SCoords {
   double z, y, x_in, nu;
 };
 
-// functions.glsl:781-787 (u_r), as GL texel-space z.
-ATMO_HD double s_r_texel(const Job& j, double r) {
-  double rho = safe_sqrt(r * r - j.rb * j.rb);
-  return unit_to_texel(rho / j.H, j.nr);
-}
-
-// rb^2 as a rounded product, never part of a fused multiply-add: where a ray
-// grazes the ground, the discriminant below and rho^2 are differences of nearly
-// equal squares, and a lookup moves by percents if only one of them is rounded.
-ATMO_HD double rb_squared(const Job& j) {
+// a^2 as a rounded product, never part of a fused multiply-add, if kRounded.
+//
+// Where a ray grazes the ground, and where a lookup's radius is clamped to the
+// ground's, rho^2 and the discriminant of s_mu_texel are differences of (nearly) equal
+// squares. With all squares rounded rho is 0 at r = rb; with one fused it may be 6e-5,
+// and a lookup below the ground then reads the other half of the mu axis. Which are
+// fused depends on what else a kernel computes, so the lookups round them.
+//
+// GetSkyRadianceToPoint rounds rb^2 only (kRounded false), which keeps the values it
+// has always had. They are right except for segments that pass below the ground and
+// whose light shaft ends there, where rb^2 rounds down: 100 to 150 of 2.07M scattered
+// rays with shafts, at about half of all radii.
+ATMO_HD double rounded_square(double a) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-  return j.rb * j.rb;
+  return a * a;
+}
+template <bool kRounded>
+ATMO_HD double squared(double a) {
+  return kRounded ? rounded_square(a) : a * a;
+}
+
+// functions.glsl:781-787 (u_r), as GL texel-space z.
+template <bool kRounded = true>
+ATMO_HD double s_r_texel(const Job& j, double r) {
+  double rho = safe_sqrt(squared<kRounded>(r) - rounded_square(j.rb));
+  return unit_to_texel(rho / j.H, j.nr);
 }
 
 // functions.glsl:789-812 (u_mu), as GL texel-space y. The ground and sky
 // halves each map to MU/2 texels.
+template <bool kRounded = true>
 ATMO_HD double s_mu_texel(const Job& j, double r, double mu, bool ground) {
-  double rho = safe_sqrt(r * r - j.rb * j.rb);
+  double rho = safe_sqrt(squared<kRounded>(r) - rounded_square(j.rb));
   double r_mu = r * mu;
-  double disc = r_mu * r_mu - r * r + rb_squared(j);
+  double disc = squared<kRounded>(r_mu) - squared<kRounded>(r) + rounded_square(j.rb);
   const int half = j.nmu / 2;
   double u_mu;
   if (ground) {
@@ -433,11 +448,12 @@ ATMO_HD double s_mus_texel(const Job& j, double mu_s) {
 
 // functions.glsl:773-831, with u_nu expressed as the nu slice coordinate
 // u_nu * (NU - 1) of functions.glsl:967.
+template <bool kRounded>
 ATMO_HD SCoords s_coords(const Job& j, double r, double mu, double mu_s,
                          double nu, bool ground) {
   SCoords c;
-  c.z = s_r_texel(j, r);
-  c.y = s_mu_texel(j, r, mu, ground);
+  c.z = s_r_texel<kRounded>(j, r);
+  c.y = s_mu_texel<kRounded>(j, r, mu, ground);
   c.x_in = s_mus_texel(j, mu_s);
   c.nu = (nu + 1.0) / 2.0 * (j.nnu - 1);
   return c;

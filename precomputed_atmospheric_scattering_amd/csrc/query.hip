@@ -142,7 +142,7 @@ __device__ __forceinline__ void lookup_lines(const Job& J, const SCoords& c, uin
   *m = as_d4(am);
 }
 
-// functions.glsl:1658-1690. kF32: FP32 tap weights and sums (lookups whose
+// functions.glsl:1658-1690. kF32: FP32 tap weights and sums (GetSkyRadiance, whose
 // result is not a difference of two lookups); otherwise FP64. kSeparate: S and
 // SM are separate. kLines: they may have a lookup copy; then all lanes of the wave
 // call it, with the wave's kStageParts parts of LDS.
@@ -150,7 +150,7 @@ template <bool kF32, bool kSeparate, bool kLines>
 __device__ D4 combined_scattering(const Job& J, double r, double mu, double mu_s,
                                   double nu, bool ground, uint4* stage, D4* single_mie) {
   using Real = typename std::conditional<kF32, float, double>::type;
-  const SCoords c = s_coords(J, r, mu, mu_s, nu, ground);
+  const SCoords c = s_coords<kF32>(J, r, mu, mu_s, nu, ground);
   auto lookup = [&](const auto& lut) {
     return kF32 ? s_lookup_f(J, lut, c) : s_lookup_d(J, lut, c);
   };
