@@ -155,29 +155,44 @@ struct DeviceArrays {
   }
 };
 
-// Times every shape of the passes asked for on k copies of the tuning
-// atmosphere at sizes z; writes the fastest shapes.
-atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStream_t s,
-                      int* sd_out, MsShape* ms_out) {
-  const Sizes z = sizes_of(lz);
-  const double texels = static_cast<double>(z.s_texels());
+// The tuning atmosphere at sizes lz, in as many copies as fill the GPU, with the
+// deltas of orders 1 and 2: every input of the timed launches.
+struct TuneModels {
+  std::vector<std::unique_ptr<atmo_model, void (*)(atmo_model*)>> owned;
+  std::vector<atmo_model*> models;
+};
+atmo_status make_models(const atmo_lut_sizes& lz, bool half, hipStream_t s, TuneModels* out) {
+  const double texels = static_cast<double>(sizes_of(lz).s_texels());
   const int k = std::max(1, std::min(kMaxCopies, static_cast<int>(std::ceil(kTuneTexels /
                                                                                texels))));
   const EarthParams ep;
-  const atmo_model_params p = ep.params();
-  std::vector<std::unique_ptr<atmo_model, void (*)(atmo_model*)>> owned;
-  std::vector<atmo_model*> models;
+  atmo_model_params p = ep.params();
+  p.half_precision = half ? 1 : 0;
   for (int i = 0; i < k; ++i) {
     atmo_model* m = nullptr;
     ATMO_TRY(atmo_model_create(&p, &lz, &m));
-    owned.emplace_back(m, [](atmo_model* x) { (void)atmo_model_destroy(x); });
-    models.push_back(m);
+    out->owned.emplace_back(m, [](atmo_model* x) { (void)atmo_model_destroy(x); });
+    out->models.push_back(m);
     m->retain = true;  // keep the deltas: the timed launches read them
   }
-  // Orders 1 and 2 give every input of the timed launches: the delta
-  // scattering, irradiance and density LUTs.
   std::vector<unsigned> orders(k, 2);
-  ATMO_TRY(atmo_model_init_batch(models.data(), orders.data(), k, s));
+  return atmo_model_init_batch(out->models.data(), orders.data(), k, s);
+}
+
+// Times every shape of the passes asked for; writes the fastest shapes. The
+// multiple-scattering shapes are timed on FP32-storage models, which all use them,
+// the density's on models whose density takes the shapes (sd_uses_tile): FP16
+// storage, up to the size at which that sums by directions in all orders, and FP32
+// storage beyond it, which does at order 2.
+atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStream_t s,
+                      int* sd_out, MsShape* ms_out) {
+  const Sizes z = sizes_of(lz);
+  const bool sd_half = static_cast<int64_t>(z.s_texels()) <= atmo::kFixedTexels;
+  TuneModels f32, f16;
+  if (do_ms || !sd_half) ATMO_TRY(make_models(lz, false, s, &f32));
+  if (do_sd && sd_half) ATMO_TRY(make_models(lz, true, s, &f16));
+  const std::vector<atmo_model*>& sd_models = sd_half ? f16.models : f32.models;
+  const int k = static_cast<int>((do_ms ? f32 : do_sd && sd_half ? f16 : f32).models.size());
 
   DeviceArrays d;
   TUNE_HIP(device_malloc(&d.jobs, k * sizeof(atmo::Job)));
@@ -185,7 +200,10 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
   TUNE_HIP(hipEventCreate(&d.start));
   TUNE_HIP(hipEventCreate(&d.stop));
   const int w = z.nnu * z.nmus;
-  auto time_pass = [&](Pass pass, int tile, int row_order, float* best) -> atmo_status {
+  // 'order' is the order of the density.
+  auto time_pass = [&](Pass pass, int order, int tile, int row_order,
+                       float* best) -> atmo_status {
+    const std::vector<atmo_model*>& models = pass == kSD ? sd_models : f32.models;
     std::vector<atmo::Job> js(k);
     std::vector<int> fb(k + 1);
     int total = 0;
@@ -193,6 +211,8 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
       js[i] = models[i]->jobs[0];
       (pass == kSD ? js[i].sd_tile : js[i].ms_tile) = tile;
       if (pass == kMS) js[i].ms_row_order = row_order;
+      js[i].ms_paired = atmo::ms_pairs(js[i]) ? 1 : 0;
+      js[i].ms_spread_out = atmo::ms_spread(js[i]) ? 1 : 0;
       fb[i] = total;
       total += pass_blocks(pass, js[i]);
     }
@@ -211,7 +231,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     pl.min_w = w;
     pl.max_lds_w = w <= atmo::kMsMaxRow ? w : 0;
     pl.kinds = atmo::kJobsF32;
-    pl.dj_kinds = atmo::kDjF32;
+    pl.dj_kinds = atmo::dj_kind(js[0]);
     pl.ss_kinds = 0;
     pl.ss_lds = 0;
     pl.sd_kinds = 1 << atmo::sd_split(js[0]);
@@ -219,7 +239,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     pl.arc_lds = 0;
     pl.tile = tile;
     auto launch = [&]() {
-      return pass == kSD ? atmo::launch_scattering_density(pl, 2, s)
+      return pass == kSD ? atmo::launch_scattering_density(pl, order, s)
                          : atmo::launch_multiple_scattering(pl, s);
     };
     ATMO_TRY(check_launch(launch(), "tuning launch"));  // warm-up
@@ -242,11 +262,20 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
     return t[dflt] >= kMinGain * t[best] ? best : dflt;
   };
   if (do_sd) {
-    std::vector<double> t(atmo::kSdTiles);
-    for (int tile = 0; tile < atmo::kSdTiles; ++tile) {
-      float ts = 0.0f;
-      ATMO_TRY(time_pass(kSD, tile, 0, &ts));
-      t[tile] = ts;
+    // The orders >= 3 are one kernel: for the default 4 orders, two launches of it to
+    // one of order 2's. (Where they are arc sums order 2 decides.)
+    std::vector<double> t(atmo::kSdTiles, 0.0);
+    for (int order = 2; order <= 3; ++order) {
+      if (!atmo::sd_uses_tile(sd_models[0]->jobs[0], order)) {
+        if (order == 2)
+          return fail(ATMO_ERROR_INVALID_ARGUMENT, "tuning models without density shapes");
+        continue;
+      }
+      for (int tile = 0; tile < atmo::kSdTiles; ++tile) {
+        float ts = 0.0f;
+        ATMO_TRY(time_pass(kSD, order, tile, 0, &ts));
+        t[tile] += order == 2 ? ts : 2.0 * ts;
+      }
     }
     *sd_out = pick(t, atmo::sd_default_tile(z.nmu, z.nnu));
   }
@@ -262,7 +291,7 @@ atmo_status tune_size(const atmo_lut_sizes& lz, bool do_sd, bool do_ms, hipStrea
       if (w > atmo::kMsMaxRow && tile != dflt.tile) continue;
       for (int o = 0; o < kO; ++o) {
         float tm = 0.0f;
-        ATMO_TRY(time_pass(kMS, tile, o, &tm));
+        ATMO_TRY(time_pass(kMS, 0, tile, o, &tm));
         t[kO * tile + o] = tm;
       }
     }

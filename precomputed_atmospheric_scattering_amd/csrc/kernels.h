@@ -123,6 +123,12 @@ ATMO_HD int sd_split(const Job& j) {
   return i;
 }
 
+// Whether the density of an order takes the job's tile shape (kSdTile): the directions
+// with a thread per output.
+ATMO_HD bool sd_uses_tile(const Job& j, int order) {
+  return order == 2 ? sd_split(j) == kSdSplits : !arc_sums(j);
+}
+
 // Single scattering: blocks of 'block' texels of a packed row, for 'nit'
 // iterations of a model. Where 'staged', the block blends the transmittance
 // rows of each sample in LDS for ss_rows of them; otherwise every texel gathers

@@ -1493,19 +1493,30 @@ void plan_levels(atmo_model* const* models, const unsigned* orders, int count,
     l.total_blocks = total;
     plan->levels.push_back(l);
   };
-  // Scattering density of order 2 and multiple scattering: one launch per tile shape
-  // among the jobs (each kernel instance has one shape).
+  // Scattering density by directions and multiple scattering: one launch per tile
+  // shape among the jobs that use it (each kernel instance has one shape). The other
+  // density jobs join the first of them.
   auto add_level = [&](Pass p, int order, const std::vector<std::pair<int, int>>& sel) {
     if (p != kSD && p != kMS) {
       add_one(p, order, 0, sel);
       return;
     }
     const int ntiles = p == kSD ? atmo::kSdTiles : atmo::kMsTiles;
+    auto job = [&](const std::pair<int, int>& mj) -> const atmo::Job& {
+      return models[mj.first]->jobs[mj.second];
+    };
+    int first = ntiles;
+    for (const auto& mj : sel)
+      if (p == kSD && atmo::sd_uses_tile(job(mj), order))
+        first = std::min(first, job(mj).sd_tile);
+    if (first == ntiles) first = 0;
     for (int t = 0; t < ntiles; ++t) {
       std::vector<std::pair<int, int>> part;
       for (const auto& mj : sel) {
-        const atmo::Job& j = models[mj.first]->jobs[mj.second];
-        if ((p == kSD ? j.sd_tile : j.ms_tile) == t) part.push_back(mj);
+        const atmo::Job& j = job(mj);
+        const int tile = p == kMS ? j.ms_tile
+                                  : (atmo::sd_uses_tile(j, order) ? j.sd_tile : first);
+        if (tile == t) part.push_back(mj);
       }
       add_one(p, order, t, part);
     }
