@@ -74,6 +74,12 @@ typedef struct atmo_model_params {
   double length_unit_in_meters;
   unsigned num_precomputed_wavelengths;
   int combine_scattering_textures;
+  /* FP16 storage of the scattering LUTs. The tables of models of up to 2^22
+   * scattering texels keep their bits from one version of the library to the
+   * next, on the same GPU; for that they are summed by kernels that take up
+   * to 2.4 times the time of an FP32 model's on the smallest grids and a
+   * quarter more at the default sizes. Of larger ones the last bit of a texel
+   * may change. */
   int half_precision;
 } atmo_model_params;
 

@@ -65,14 +65,25 @@ ATMO_HD int sd_default_tile(int nmu, int nnu) {
   return nmu * ((nnu + 3) / 4) <= 256 ? 3 : 0;
 }
 
-// FP16-storage models of up to kFixedTexels texels keep the order in which
-// their sums of float32 were always made. FP16 rounding turns a difference of
-// 1e-7 of a sum into one of 1e-3 in some texels (arc sums for the orders >= 3:
-// the last bit of 9e-5 of the texels at 1.05M), and GetSkyRadianceToPoint, a
-// difference of two lookups, into up to 4e-3 of the rms radiance: within the
-// format's error, but a model then shades differently from LUT files and from
-// other models made before. Beyond that size the time decides: at 16.8M texels
-// and 8 orders the arc sums save 57 ms of 212, at 1.05M and 4 orders 1.4 of 6.2.
+// FP16-storage models of up to kFixedTexels texels keep the bits of their tables
+// (half_precision in include/atmo.h): the order in which their sums of float32 were
+// always made. FP16 rounding turns a difference of 1e-7 of a sum into the last bit of
+// 9e-5 of the texels (arc sums for the orders >= 3, 1.05M texels), and
+// GetSkyRadianceToPoint, a difference of two lookups, that into up to 4e-3 of the rms
+// radiance: within the format's error, but a model would shade differently from LUT
+// files and models made before. The price, ms per Init by directions | arcs and split
+// order 2, on MI355X:
+//   texels    3 wavelengths, 4 orders   15, 4          15, 8
+//   8192      .77 | .33                 .81 | .46      1.6 | .84
+//   262144    .89 | .58                 2.0 | 1.6      3.7 | 2.6
+//   1.05M     1.54 | 1.35               6.2 | 4.9      12.1 | 8.2
+//   2.1M      2.7 | 2.4                 12.5 | 9.8     24.2 | 16.5
+//   4.2M      5.2 | 4.7                 24.3 | 19.3    48.0 | 32.9
+//   8.4M      9.8 | 8.9                 47.5 | 37.8    94.0 | 66.8
+//   16.8M     20.1 | 19.5               96.6 | 78.9    193 | 140
+// The share is much the same at every size, so the line is no crossover: it is where
+// 8 orders cost 15 ms more, at four times the default sizes. A table beyond it takes
+// the time, up to 53 ms, and its last bits are not promised.
 constexpr int64_t kFixedTexels = int64_t{1} << 22;
 ATMO_HD bool fixed_sums(const Job& j) {
   return j.half_luts != 0 &&

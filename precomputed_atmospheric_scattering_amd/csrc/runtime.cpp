@@ -282,9 +282,9 @@ void free_temporaries(atmo_model* m) {
 namespace {
 
 // The block of temporaries that the last Init on a device gave back, for the
-// next one: mapping and unmapping 46 MB (reference sizes, 3 wavelengths) took
-// 0.19 ms of an Init of 1.45 ms on MI355X, 568 MB (15) 0.7 ms of 5.7, and a
-// hipFree at times 7 ms. At most one block of at most kPooledBytes is kept per
+// next one: mapping and unmapping 46 MB (reference sizes, 3 wavelengths) takes
+// 0.055 ms of an Init of 1.40 ms on MI355X, 568 MB (15) 0.42 ms of 5.43, and a
+// hipFree took 7 ms at times. At most one block of at most kPooledBytes is kept per
 // device. It is freed when no model is left, when an allocation of the library
 // finds no memory, and when a larger one takes its place.
 constexpr size_t kPooledBytes = size_t{1} << 30;
