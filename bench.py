@@ -52,11 +52,11 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X FP32 vector (packed FMA = 2 flops per lane)
 # or one packed). Every VALU instruction of a wave counts 64 lane-ops.
 PEAK_VALU_TOPS = PEAK_FP32_TFLOPS / 2.0
 # FP arithmetic (add, mul, FMA) lane-instructions per second when they issue
-# one per SIMD per 4 clocks: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz. On
-# MI355X two FP32 arithmetic instructions do not issue together (csrc/
-# peaks.hip measures FMA + add pairs at the single rate, FMA + integer or
-# conversion pairs at twice it), and packed FP32 is not used here, so this
-# is the ceiling of a kernel made of FP32 (or FP64) arithmetic.
+# one per SIMD per 4 clocks: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz. csrc/
+# peaks.hip measures an FMA + add mix at this rate and FMA + integer or
+# conversion mixes at twice it. It is a scale, not a hard ceiling: the order-2
+# density issues FP32 arithmetic at 1.08 of it, so some of its instructions do
+# issue together.
 PEAK_FP_ARITH_TOPS = 256 * 4 * 16 * 2.4e9 / 1e12
 PEAK_HBM_GBS = 8000.0
 # Algorithmic work per integration sample (VALU lane-ops, transcendentals

@@ -25,7 +25,8 @@
 //
 // Per texel and angle there are about 2 + 2/3 NU terms (11 at NU = 16, 6 at 8)
 // instead of 32 azimuths, and their G serve all wavelengths of the model.
-// Against the kernel that interpolated per direction, wavelength triple and
+// (With one iteration and many NU the directions are faster: arc_sums.) Against the
+// kernel that interpolated per direction, wavelength triple and
 // texel (its FP32 arithmetic issued at 0.98 of the ceiling), per order, on
 // MI355X:
 //   texels, wavelengths          direction by direction   arcs
@@ -33,8 +34,8 @@
 //   16.8M (NU 16), 3             2.99 ms                  2.93 ms
 //   1.05M (NU 8), 15             0.92 ms                  0.21 ms
 //   1.05M (NU 8), 3              0.23 ms                  0.146 ms
-// With 15 wavelengths it issues vector or matrix instructions in 87% of the
-// cycles; with 3, vector ones in 80% with the LDS 75% busy.
+// At 16.8M texels with 15 wavelengths vector instructions issue in 61% of the
+// cycles, the matrix units are busy 28%, and the LDS is busy 55%.
 //
 // The outgoing phase function is Rayleigh's plus Mie's with a factor per
 // wavelength, so there are two G per term and two sums, combined at the end.

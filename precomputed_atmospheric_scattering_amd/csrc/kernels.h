@@ -94,7 +94,7 @@ ATMO_HD bool fixed_sums(const Job& j) {
 // direction by direction. The arcs' terms serve all iterations of a model, and are
 // 2 + 2/3 NU in number: with one iteration and many NU the directions are faster.
 // Measured on MI355X, ms per order, 3 wavelengths, directions | arcs:
-//   NU 16, 16.8M texels 2.9 | 2.8;  NU 20, 2.6M .55 | .54, 5.2M .99 | 1.07
+//   NU 16, 8.4M texels 1.43 | 1.32;  NU 20, 2.6M .55 | .54, 5.2M .99 | 1.07
 //   NU 24, 1.6M .42 | .40, 2.0M .42 | .48, 3.1M .60 | .73, 12.6M 2.24 | 2.88
 //   NU 32, 2.1M .45 | .49, 8.4M 1.66 | 1.89
 // With 6 wavelengths the arcs are 1.4 times as fast at the least.
