@@ -146,13 +146,21 @@ ATMO_HD bool sd_uses_tile(const Job& j, int order) {
 // its four transmittance texels.
 //
 // A staged block blends all TW columns for each sample, however few texels it
-// has, and has a barrier per sample. It is worth that where the texels are at
-// least a quarter of the columns, the waves of a block are mostly full, and two
-// blocks per CU hide the barriers. Measured on MI355X (ms; wl: wavelengths),
-// gathered | staged:
-//   row of 256, TW 256, 3 wl: 4096 rows .147 | .131, 256 rows .024 | .031
-//   row of 192, TW 256, 3 wl: 1344 rows .054 | .053; 128: 2048 rows .052 | .066
-//   row of 512, 2048 rows, 3 wl: TW 2048 .305 | .252, TW 4096 .357 | .69
+// has, and has a barrier per sample: 2 columns a thread are worth it, or 4 in
+// blocks of 512 that serve several iterations. Rows of 513..768 texels, which
+// leave a third of 512-thread blocks idle, take blocks of 256 while TW is 2 columns
+// a thread. Gathering blocks of one iteration run three to a CU, so up to
+// kSsGatherBlocks of them are a single round that staging does not shorten;
+// from 3 iterations on it does, at 512. Measured on MI355X (ms; wl:
+// wavelengths), gathered | staged:
+//   row of 256, TW 256, 3 wl: 4096 rows .147 | .131, 512 rows .028 | .034
+//   row of 512, TW 256, 3 wl: 384 rows .038 | .041, 400 rows .045 | .040; 15 wl:
+//     192 rows .092 | .118, 256 rows .112 | .119, 496 rows .210 | .170
+//   row of 297, TW 256, 15 wl: 192 rows .090 | .098, 256 rows .113 | .101
+//   row of 600, TW 256, 432 rows, 15 wl: .240 | .229 (256 threads), .308 (512);
+//     row of 768, TW 256, 512 rows, 6 wl: .161 | .117 (256), .141 (512)
+//   row of 256, TW 1024, 9 wl: 800 rows .152 | .220; row of 512, TW 2048, 3 wl:
+//     400 rows .060 | .075
 //   row of 65, 16128 rows, TW 4096: .34 | 9.0 (3 wl), 1.8 | 50 (15 wl)
 // Iterations share a block that gathers where three blocks per CU are left and
 // the lines that the block reads per sample, in each iteration 2 rows of at most
@@ -161,9 +169,8 @@ ATMO_HD bool sd_uses_tile(const Job& j, int order) {
 // row of 32, TW 256, 15 wl: 2048 rows .126 | .117, 512 rows .046 | .069.
 constexpr int kSsIters = 5;
 constexpr int kSsRowBytes = 64 << 10;  // at most, if iterations share a block
-constexpr int kSsStagedWidth = 192;    // shortest row
-constexpr int kSsColumns = 4;          // at most, blended per texel
-constexpr int kSsStagedBlocks = 512;
+constexpr int kSsStagedWidth = 160;    // shortest row
+constexpr int kSsStagedBlocks = 512;   // of 256 texels, 3 iterations or more
 constexpr int kSsGatherBlocks = 768;
 constexpr int kSsGatherBytes = 24 << 10;
 constexpr ATMO_HD int ss_rows(int nit, bool staged) { return !staged ? 0 : (nit < 3 ? 1 : 2); }
@@ -181,10 +188,13 @@ struct SsTiling {
   bool fixed;  // FP32 job of fixed_sums: k_single_scattering_fixed instead
   ATMO_HD explicit SsTiling(const Job& j) {
     const int w = j.nnu * j.nmus, most = j.niter < kSsIters ? j.niter : kSsIters;
-    const int wide = w > kBlock ? 2 * kBlock : kBlock;
+    const bool thirds = w > 2 * kBlock && w <= 3 * kBlock && j.tw <= 2 * kBlock;
+    const int wide = w > kBlock && !thirds ? 2 * kBlock : kBlock;
+    const int columns = most > 1 ? (wide > kBlock ? 4 : 2) * wide
+                                 : 2 * (w < kBlock ? w : wide);
     fixed = fixed_sums(j) && !j.acc64;
-    staged = w >= kSsStagedWidth && j.tw <= kSsColumns * (w < wide ? w : wide) &&
-             blocks(j, wide) >= kSsStagedBlocks &&
+    staged = w >= kSsStagedWidth && j.tw <= columns &&
+             blocks(j, kBlock) >= (most > 2 ? kSsStagedBlocks : kSsGatherBlocks + 1) &&
              (most == 1 || ss_row_bytes(j, most, true) <= kSsRowBytes);
     block = staged ? wide : (w > 64 ? kBlock : 64);
     const int lines = (j.tw + 7) / 8 < w ? (j.tw + 7) / 8 : w;  // 8 texels each

@@ -33,7 +33,7 @@ BATCHES = {
     "storage": [(config(64, 8, 64, 16, 4, 3, True), 4), (config(64, 8, 64, 16, 4, 3), 4),
                 (config(64, 5, 46, 9, 7, 15, True), 3), (config(64, 64, 128, 64, 9, 3, True), 3),
                 (config(64, 32, 128, 24, 20), 3), (config(64, 2, 4, 2, 2, 3, True), 5)],
-    "rows": [(config(256, 16, 34, 32, 8), 3), (config(64, 4, 10, 73, 7, 3, True), 3),
+    "rows": [(config(256, 16, 50, 32, 8), 3), (config(64, 4, 10, 73, 7, 3, True), 3),
              (config(64, 4, 10, 64, 17, 6), 3), (config(64, 32, 64, 64, 10), 2),
              (config(64, 8, 34, 4, 2, 15, True), 4), (config(64, 41, 70, 9, 3, 15, True), 2)],
 }

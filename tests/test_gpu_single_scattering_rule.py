@@ -21,13 +21,23 @@ pytestmark = pytest.mark.gpu
 
 # TW, R, MU, MU_S, NU, wavelengths.
 CASES = [
-    # Rows of 190 (gathered) and 192 texels; TW of 4 columns a texel and beyond.
+    # Rows of 190 and 192 texels, gathered; TW of 4 columns a texel and beyond.
     (64, 16, 32, 95, 2, 3), (64, 16, 32, 48, 4, 3),
     (768, 16, 32, 48, 4, 3), (769, 16, 32, 48, 4, 3), (768, 16, 32, 48, 4, 15),
     # Wide transmittance over short and long rows.
     (4096, 4, 16, 13, 5, 3), (4096, 4, 16, 13, 5, 15), (4096, 2, 8, 64, 16, 15),
-    # 510 blocks and 512.
-    (64, 15, 34, 32, 8, 3), (64, 16, 32, 32, 8, 3),
+    # Few blocks: 510, 512; with 3 iterations staged from 512 on.
+    (64, 15, 34, 32, 8, 3), (64, 16, 32, 32, 8, 3), (64, 15, 34, 32, 8, 9),
+    (64, 16, 32, 32, 8, 9),
+    # 768 blocks gather, 780 stage; rows of 160 on; 2 columns a texel and beyond.
+    (64, 16, 48, 32, 8, 3), (64, 15, 52, 32, 8, 3), (64, 15, 52, 40, 4, 3),
+    (384, 15, 52, 48, 4, 3), (385, 15, 52, 48, 4, 3),
+    # Rows of 513..768: 256 threads to TW 512, then 512.
+    (512, 8, 34, 57, 9, 3), (513, 8, 34, 57, 9, 3), (512, 6, 30, 64, 12, 15),
+    (513, 6, 30, 64, 12, 15),
+    # Blocks of 512: 2 columns a thread, 4 with 2 iterations, the LDS of more.
+    (1024, 10, 40, 33, 8, 3), (1025, 10, 40, 33, 8, 3), (2048, 10, 40, 33, 8, 6),
+    (2048, 10, 40, 33, 8, 9),
     # Gathered by 256 threads, iterations alone and shared (768 blocks).
     (64, 12, 64, 13, 5, 15), (64, 12, 62, 13, 5, 15), (512, 12, 64, 13, 5, 15),
     (64, 12, 64, 13, 5, 6), (64, 12, 64, 13, 5, 18), (96, 24, 32, 8, 4, 9),

@@ -44,19 +44,38 @@ JOBS = [job(tw, nr, nmu, nmus, nnu, niter)
 
 
 def test_staged_blocks_blend_no_more_than_they_save(rules):
-    # A staged block blends TW columns per sample and iteration for its texels.
+    # A staged block blends TW columns per sample and iteration for its texels; up to
+    # 768 blocks of one or two iterations that gather are one round of three per CU.
     staged = 0
     for (tw, _, nr, nmu, nmus, nnu, _, niter, _, _, _), r in zip(JOBS, rules(JOBS)):
         block, stage, nit, _, lds = r[:5]
         w = nmus * nnu
         if stage:
             staged += 1
-            assert tw <= 4 * min(w, block) and w >= 192 and lds <= 64 << 10
-            assert nr * nmu * -(-w // block) >= 512
+            assert tw <= (4 if niter > 1 and block > 256 else 2) * block
+            assert w >= 160 and lds <= 64 << 10
+            gathering = nr * nmu * -(-w // 256)
+            assert gathering >= 512 and (niter > 2 or gathering > 768)
         else:
             assert lds == 0 and block <= 256
         assert block >= 64 and nit in (1, niter if niter < 5 else 5)
     assert 0 < staged < len(JOBS)
+
+
+def test_staged_blocks_fit_their_rows(rules):
+    # Rows of 513..768 texels take 256-thread blocks; 2 columns a thread, or 4 in
+    # blocks of 512 that serve several iterations.
+    jobs = [job(nmus=w // 4, nnu=4, tw=tw, niter=n) for w, tw, n in (
+        (156, 256, 1), (160, 256, 1), (192, 512, 1), (256, 512, 1), (256, 513, 5), (260, 1024, 1),
+        (260, 1025, 1), (260, 2048, 2), (512, 512, 1), (516, 512, 1), (768, 512, 5),
+        (768, 513, 5), (772, 512, 1))]
+    assert [r[:2] for r in rules(jobs)] == [
+        (256, 0), (256, 1), (256, 0), (256, 1), (256, 0), (512, 1), (256, 0), (512, 1), (512, 1),
+        (256, 1), (256, 1), (512, 1), (512, 1)]
+    # 768 and 780 blocks of 256; 510 and 512.
+    jobs = [job(nr=16, nmu=48), job(nr=15, nmu=52), job(nr=15, nmu=34, niter=5),
+            job(nr=16, nmu=32, niter=5), job(nr=16, nmu=32, niter=2)]
+    assert [r[1] for r in rules(jobs)] == [0, 1, 0, 1, 0]
 
 
 def test_iterations_are_served_once(rules):
